@@ -185,7 +185,8 @@ int ttfa_varlen_bwd(const void *q, const void *k, const void *v, const void *o,
  *   workspace         : ttfa_decode_workspace_bytes(...) bytes, 16-byte aligned (fp32
  *                       per-split partials; overwritten)
  * Supported: D in {64, 128}, Hq % Hkv == 0, (Hq / Hkv) * Tq <= 32 (TTFA_E_QROWS),
- * B, Tq, max_seqlen >= 1.  Two launches on hip_stream (split pass, merge pass).
+ * B, Tq, max_seqlen >= 1.  One launch on hip_stream, or two (split pass, merge pass) where
+ * the keys of a head are split over workgroups.
  */
 long long ttfa_decode_workspace_bytes(int B, int Hq, int Hkv, int Tq, int max_seqlen, int D);
 

@@ -56,6 +56,32 @@ def test_decode_matches_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
     assert_close_abs("LSE", lse.cpu()[fin], want_lse[fin], TOL_LSE)
 
 
+@pytest.mark.parametrize("B, Hq, Hkv, Tq, Lmax, D, lens", [
+    (3, 4, 2, 1, 512, 128, [512, 33, 0]),       # 16 blocks: one workgroup per head, one launch
+    (2, 4, 2, 3, 513, 128, [513, 2]),           # 17 blocks: split, two waves per workgroup
+    (2, 2, 1, 1, 512, 64, [511, 480]),
+    (1, 2, 1, 2, 545, 64, [545]),               # D = 64 split: four waves per workgroup
+    (4, 16, 16, 1, 2017, 128, [2017, 2016, 1, 600]),   # 64 * 64 blocks: the last two-wave shape
+    (4, 16, 16, 1, 2049, 128, [2049, 31, 2048, 97]),   # 64 * 65 blocks: four waves
+    (40, 8, 8, 4, 700, 128, [700 - 17 * i for i in range(40)]),  # 320 heads: one chunk each
+    (2, 32, 1, 1, 1000, 128, [1000, 65]),       # 32 query columns fill the merge stage
+    (1, 8, 2, 8, 16500, 64, [16391]),           # many chunks of two blocks per head
+])
+def test_decode_splits_match_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
+    """Both sides of every rule that picks a call's workgroups per head and waves per
+    workgroup, with uneven and empty caches."""
+    announce(f"decode splits B={B} Hq={Hq} Hkv={Hkv} Tq={Tq} Lmax={Lmax} D={D} lens={lens[:4]}")
+    q, k, v = _inputs(B, Hq, Hkv, Tq, Lmax, D)
+    lens_t = torch.tensor(lens, dtype=torch.int32)
+    want_o, want_lse = decode_reference(q, k, v, lens)
+    o, lse = flash_attn_decode(q.to(DEV), k.to(DEV), v.to(DEV), lens_t.to(DEV))
+    assert_close_abs("O", o.cpu(), want_o, TOL[torch.bfloat16])
+    torch.cuda.synchronize()
+    seen = torch.isfinite(want_lse)
+    assert torch.equal(torch.isfinite(lse.cpu()), seen)
+    assert_close_abs("lse", lse.cpu()[seen], want_lse[seen], TOL_LSE)
+
+
 def test_decode_agrees_with_forward_kernel():
     announce("decode vs batched forward last rows")
     B, Hq, Hkv, T, D, Tq = 2, 8, 2, 700, 128, 2

@@ -7,20 +7,35 @@
 // last Tq rows: query i of the new tokens sits at position L_b - Tq + i and sees keys
 // 0 .. L_b - Tq + i of the cache, O = softmax(q k^T * scale) v, LSE = m + ln(l).
 //
-// Work split (split-K, "flash decoding"): the cache of every (batch, KV head) is cut into
-// ranges of `wkeys` keys, one range per wave; a 256-thread workgroup runs 4 ranges.  All
-// G query heads of the KV head and all Tq rows form the R = G * Tq <= 32 query columns
-// of one 32x32 MFMA tile (columns past R repeat valid ones and are not stored), so the K
-// and V bytes of a range are read once for the whole group.  A wave streams its range in
-// 32-key blocks: the block's K fragments load straight into the MFMA A-operand registers
-// (row-major rows are the A layout), V goes into a wave-private, swizzled, double-
-// buffered LDS block for the transposed operand reads, and the next block's loads are in
-// flight while the current one is computed (the wave waits on its own vmcnt only; no
-// workgroup barriers).  Per block: S^T = K Q^T, online softmax in the exp2 domain
-// (lazy rescale as in the forward kernel), O^T += V^T P^T.  Each wave writes an fp32
-// partial (unnormalised O, running max m in log2 units, sum l) per query row; a second
-// kernel merges the partials of a row with the log-sum-exp rule.  The memory traffic is
-// the cache bytes (the roofline of decode), read once.
+// Work split (split-K, "flash decoding"): a unit is one (batch, KV head).  Its 32-key blocks
+// in use (its own cache length, not the capacity) are dealt evenly to n_chunks workgroups,
+// and a workgroup's blocks to its waves in turn, so the workgroups of a unit have the same
+// work whatever its length.  Workgroups are numbered chunk-major: consecutive ids, which
+// the hardware deals to the XCDs, are different units, so batches of uneven lengths spread
+// over all XCDs.  All G query heads of the KV head and all Tq rows form the R = G * Tq <= 32
+// query columns of one 32x32 MFMA tile (columns past R repeat valid ones and are not
+// stored), so the K and V bytes are read once for the whole group.
+//
+// Data path: a wave loads a block's K and V rows straight into its own LDS stage, whole
+// rows in order (16 bytes per lane, 1 KB per instruction), the next block's loads in flight
+// while the current one is computed (the wave waits on its own vmcnt only; no workgroup
+// barriers).  K fragments loaded straight into the MFMA operand registers, 32 bytes from
+// each of 32 rows per instruction, read 8% slower at 32 x 4096 keys.  Per block:
+// S^T = K Q^T, online softmax in the exp2 domain (lazy rescale as in the forward kernel),
+// O^T += V^T P^T.  The waves' partials (unnormalised O, running max m in log2 units, sum l)
+// are merged through LDS, in wave order.  With one chunk the workgroup then writes O and
+// LSE itself; otherwise it writes one fp32 partial per query row, and a second kernel
+// merges the chunks with the log-sum-exp rule.
+//
+// What bounds it: the cache bytes from HBM (a plain read kernel reaches 6.8-7.1 TB/s on
+// MI355X), and for small caches the launches.  Back-to-back time per call, before (one
+// range of keys per wave, four partials per workgroup, always two launches) and now:
+//   B 32, Hkv 8, D 128, lengths 410..4096 of 4096: 73.0 -> 63.9 us (5.0 TB/s)
+//   B 32, Hkv 8, D 128, 4096 keys each:            98.9 -> 90.5 us (5.9 TB/s)
+//   B 1,  Hkv 8, D 128, 16384 keys:                19.5 -> 19.2 us
+//   B 64, Hkv 12, D 64, lengths 200..2000 of 2000: 51.1 -> 44.8 us
+//   B 1,  Hkv 2, D 128, 512 keys:                  11.1 ->  8.3 us (one launch)
+#include "fa_bwd.h"  // allow_lds
 #include "fa_common.h"
 #include "fa_kernels.h"
 
@@ -30,17 +45,14 @@ namespace {
 
 constexpr float kDecodeSlack = 8.0f;
 constexpr int kDecBlock = 32;  // keys per block
-constexpr int kDecWaves = 4;   // ranges (waves) per workgroup
 constexpr int kDecMaxSplits = 512;  // partials per query row, at most
-constexpr int kCombinePrefetch = 16;  // partial rows per merge thread loaded up front ...
-constexpr int kCombinePrefetchMin = 64;  // ... when a row has at least this many partials
 
 template <int D>
 struct DecShape {
   static constexpr int KK = D / 16, DB = D / 32, CH = D / 8;
-  static constexpr int VLOADS = kDecBlock * CH / 64;            // 1 KB DMA blocks per V block
-  static constexpr int VMEM_PER_BLOCK = VLOADS + KK;            // vector memory ops per block
-  static constexpr int WAVE_LDS = 2 * kDecBlock * D;            // bf16 elements, two stages
+  static constexpr int LOADS = kDecBlock * CH / 64;       // 1 KB DMA blocks per K (V) block
+  static constexpr int VMEM_PER_BLOCK = 2 * LOADS;        // vector memory ops per block
+  static constexpr int WAVE_LDS = 2 * 2 * kDecBlock * D;  // bf16 elements, [stage][K|V]
 };
 
 // s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt bits 3:0 and 15:14; expcnt, lgkmcnt at max)
@@ -52,12 +64,15 @@ __device__ __forceinline__ void wait_vmcnt() {
 
 // One 32-key block of one wave: S^T = K Q^T, mask, online softmax, O^T += V^T P^T.
 template <int D, bool MASK>
-__device__ __forceinline__ void decode_block(const bf16x8 (&kf)[D / 16], const bf16 *Vt,
+__device__ __forceinline__ void decode_block(const bf16 *Kt, const bf16 *Vt,
                                              const bf16x8 (&qf)[D / 16], f32x16 (&oacc)[D / 32],
                                              float &m_t, float &l_part, float scale_log2, int k0,
                                              int pos, int L, int lane) {
   using P = DecShape<D>;
   const int lg = lane >> 5;
+  bf16x8 kf[P::KK];
+#pragma unroll
+  for (int kk = 0; kk < P::KK; ++kk) kf[kk] = lds_read_row8<D, 1>(Kt, lane & 31, 2 * kk + lg);
   f32x16 s = mfma32(kf[0], qf[0], f32x16{});
 #pragma unroll
   for (int kk = 1; kk < P::KK; ++kk) s = mfma32(kf[kk], qf[kk], s);
@@ -106,24 +121,25 @@ __device__ __forceinline__ void decode_block(const bf16x8 (&kf)[D / 16], const b
 
 }  // namespace
 
-// Grid: B * Hkv * n_chunks workgroups of 4 waves; wave w of chunk c owns keys
-// [(4c + w) * wkeys, (4c + w + 1) * wkeys) of its (batch, KV head).  Partial rows are
-// indexed (b * Hq + h) * Tq + i, each with n_splits = 4 * n_chunks slots.
-template <int D>
-__global__ __launch_bounds__(256, 2) void fa_decode_bf16_kernel(
+// Grid: n_chunks * B * Hkv workgroups of NW waves, chunk-major.  Partial rows are indexed
+// (b * Hq + h) * Tq + i, each with n_chunks slots.
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
     const bf16 *__restrict__ Q, const bf16 *__restrict__ Kc, const bf16 *__restrict__ Vc,
-    const int *__restrict__ cache_seqlens, float *__restrict__ part_o,
-    float *__restrict__ part_ml, int B, int Hq, int Hkv, int Tq, int Lmax, int n_chunks,
-    int wkeys, float scale_log2) {
+    const int *__restrict__ cache_seqlens, bf16 *__restrict__ O, float *__restrict__ LSE,
+    float *__restrict__ part_o, float *__restrict__ part_ml, int B, int Hq, int Hkv, int Tq,
+    int Lmax, int n_chunks, float scale_log2) {
   using P = DecShape<D>;
   constexpr int KK = P::KK, DB = P::DB, CH = P::CH;
-  __shared__ __attribute__((aligned(16))) bf16 lds[kDecWaves][P::WAVE_LDS];
-  const int chunk = blockIdx.x % n_chunks, bhk = blockIdx.x / n_chunks;
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  bf16 (*lds)[P::WAVE_LDS] = reinterpret_cast<bf16 (*)[P::WAVE_LDS]>(smem);
+  __shared__ float wm[NW][32], wsum[NW][32];
+  const int n_units = B * Hkv;
+  const int chunk = blockIdx.x / n_units, bhk = blockIdx.x - chunk * n_units;
   const int b = bhk / Hkv, hk = bhk - b * Hkv;
   const int G = Hq / Hkv, R = G * Tq;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wave = wave_id(), lane = threadIdx.x & 63;
   const int lq = lane & 31, lg = lane >> 5;
-  const int split = chunk * kDecWaves + wave, n_splits = n_chunks * kDecWaves;
   const int L = min(max(cache_seqlens[b], 0), Lmax);
 
   // this lane's query column
@@ -132,8 +148,10 @@ __global__ __launch_bounds__(256, 2) void fa_decode_bf16_kernel(
   const int pos = L - Tq + i;  // last visible key of this column
   const int64_t qrow = ((int64_t)b * Hq + h) * Tq + i;
 
-  const int k_lo = split * wkeys;
-  const int k_hi = min(k_lo + wkeys, L);  // keys past L do not exist
+  // The unit's blocks in use are dealt evenly to its chunks, a chunk's blocks to its waves
+  // in turn, so every workgroup of a unit has the same work whatever the cache length.
+  const int nb = (L + kDecBlock - 1) / kDecBlock, per = (nb + n_chunks - 1) / n_chunks;
+  const int blk0 = chunk * per + wave, blk1 = min((chunk + 1) * per, nb);
   bf16 *wl = lds[wave];
 
   f32x16 oacc[DB];
@@ -141,88 +159,114 @@ __global__ __launch_bounds__(256, 2) void fa_decode_bf16_kernel(
   for (int db = 0; db < DB; ++db) oacc[db] = f32x16{};
   float m_t = -INFINITY, l_part = 0.f;
 
-  if (k_lo < k_hi) {
-    const auto rq = make_rsrc(Q + qrow * D, (uint32_t)D * 2);
+  if (blk0 < blk1) {
     const int64_t kvbase = ((int64_t)b * Hkv + hk) * Lmax * D;
-    const uint32_t kv_bytes = (uint32_t)L * D * 2;  // keys >= L read as zero
-    const auto rk = make_rsrc(Kc + kvbase, kv_bytes);
-    const auto rv = make_rsrc(Vc + kvbase, kv_bytes);
+    uint32_t koff[P::LOADS], voff[P::LOADS];  // this lane's byte offsets within a 32-row block
+#pragma unroll
+    for (int j = 0; j < P::LOADS; ++j) {
+      const int e = 64 * j + lane, row = e / CH, pc = e % CH;
+      koff[j] = (uint32_t)(row * D + swz_l<D, 1>(row, pc) * 8) * 2;
+      voff[j] = (uint32_t)(row * D + swz<D>(row, pc) * 8) * 2;
+    }
+    auto load_block = [&](int k0, int stage) {  // rows k0..k0+31 of K and V -> an LDS stage
+      bf16 *dst = wl + stage * 2 * kDecBlock * D;
+      const int64_t at = kvbase + (int64_t)k0 * D;
+      const uint32_t left = (uint32_t)(L - k0) * D * 2;  // keys >= L read as zero
+      const auto rk = make_rsrc(Kc + at, left), rv = make_rsrc(Vc + at, left);
+#pragma unroll
+      for (int j = 0; j < P::LOADS; ++j) {
+        buf_load16_lds(rk, koff[j], dst + 64 * j * 8);
+        buf_load16_lds(rv, voff[j], dst + kDecBlock * D + 64 * j * 8);
+      }
+    };
     bf16x8 qf[KK];
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
-      qf[kk] = __builtin_bit_cast(bf16x8, buf_load16(rq, (uint32_t)(16 * kk + 8 * lg) * 2));
+      qf[kk] = *reinterpret_cast<const bf16x8 *>(Q + qrow * D + 16 * kk + 8 * lg);
 
-    auto load_k = [&](bf16x8 (&kf)[KK], int k0) {
-#pragma unroll
-      for (int kk = 0; kk < KK; ++kk)
-        kf[kk] = __builtin_bit_cast(
-            bf16x8, buf_load16(rk, (uint32_t)((k0 + lq) * D + 16 * kk + 8 * lg) * 2));
-    };
-    auto load_v = [&](int k0, int stage) {  // V rows k0..k0+31 -> the wave's LDS stage
-      bf16 *dst = wl + stage * kDecBlock * D;
-#pragma unroll
-      for (int j = 0; j < P::VLOADS; ++j) {
-        const int e0 = 64 * j, e = e0 + lane, row = e / CH, pc = e % CH;
-        const uint32_t off = (uint32_t)((k0 + row) * D + swz<D>(row, pc) * 8) * 2;
-        buf_load16_lds(rv, off, dst + e0 * 8);
-      }
-    };
-
-    bf16x8 kf[KK], kn[KK];
-    load_v(k_lo, 0);
-    load_k(kf, k_lo);
-    const int n_blk = (k_hi - k_lo + kDecBlock - 1) / kDecBlock;
+    load_block(blk0 * kDecBlock, 0);
     const int first_masked = L - Tq;  // keys past this need the mask for some column
+    int stage = 0;
 #pragma unroll 1
-    for (int t = 0; t < n_blk; ++t) {
-      const int k0 = k_lo + t * kDecBlock;
-      const bool more = t + 1 < n_blk;
-      if (more) {
-        load_v(k0 + kDecBlock, (t + 1) & 1);
-        load_k(kn, k0 + kDecBlock);
-        wait_vmcnt<P::VMEM_PER_BLOCK>();  // block t's V (LDS) and K are in
+    for (int blk = blk0; blk < blk1; blk += NW, stage ^= 1) {
+      const int k0 = blk * kDecBlock;
+      if (blk + NW < blk1) {
+        load_block(k0 + NW * kDecBlock, stage ^ 1);
+        wait_vmcnt<P::VMEM_PER_BLOCK>();  // this block's K and V are in
       } else {
         wait_vmcnt<0>();
       }
       __builtin_amdgcn_sched_barrier(0);
-      const bf16 *Vt = wl + (t & 1) * kDecBlock * D;
-      if (k0 + kDecBlock - 1 > first_masked || k0 + kDecBlock > k_hi)
-        decode_block<D, true>(kf, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
+      const bf16 *Kt = wl + stage * 2 * kDecBlock * D, *Vt = Kt + kDecBlock * D;
+      if (k0 + kDecBlock - 1 > first_masked)
+        decode_block<D, true>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
       else
-        decode_block<D, false>(kf, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
-      if (more) {
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk) kf[kk] = kn[kk];
-      }
+        decode_block<D, false>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 
-  // partial of this wave's range for the columns it owns (lanes lq < R)
+  // Merge of the workgroup's waves: every wave scales its partial to the workgroup's running
+  // max and stages it as fp32 rows in its own first stage (its blocks are consumed, its loads
+  // have landed; 32 columns of D floats fill the stage), then the threads add the waves in
+  // order.
   const float l = xhalf_sum(l_part);
+  if (lg == 0) {
+    wm[wave][lq] = l > 0.f ? m_t : -INFINITY;  // a wave without visible keys weighs nothing
+    wsum[wave][lq] = l;
+  }
+  __syncthreads();
+  float M = wm[0][lq];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) M = fmax2(M, wm[w][lq]);
+  const float mw = wm[wave][lq], alpha = mw == -INFINITY ? 0.f : exp2f_fast(mw - M);
+  float *wf = reinterpret_cast<float *>(wl);
   if (lq < R) {
-    const int64_t slot = qrow * n_splits + split;
-    float *po = part_o + slot * D;
 #pragma unroll
     for (int db = 0; db < DB; ++db)
 #pragma unroll
       for (int a = 0; a < 4; ++a)
-        *reinterpret_cast<f32x4 *>(po + 32 * db + 8 * a + 4 * lg) =
-            f32x4{oacc[db][4 * a], oacc[db][4 * a + 1], oacc[db][4 * a + 2], oacc[db][4 * a + 3]};
-    if (lg == 0) *reinterpret_cast<f32x2 *>(part_ml + slot * 2) = f32x2{m_t, l};
+        *reinterpret_cast<f32x4 *>(wf + lq * D + (((8 * db + 2 * a + lg) ^ (lq & 7)) << 2)) =
+            alpha != 0.f ? f32x4{oacc[db][4 * a] * alpha, oacc[db][4 * a + 1] * alpha,
+                                 oacc[db][4 * a + 2] * alpha, oacc[db][4 * a + 3] * alpha}
+                         : f32x4{};
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < R * (D / 4); e += 64 * NW) {
+    const int c = e / (D / 4), ch = e % (D / 4);
+    f32x4 t{};
+    float mx = wm[0][c], ls = 0.f;
+#pragma unroll
+    for (int w = 1; w < NW; ++w) mx = fmax2(mx, wm[w][c]);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float *src = reinterpret_cast<const float *>(lds[w]) + c * D;
+      t += *reinterpret_cast<const f32x4 *>(src + ((ch ^ (c & 7)) << 2));
+      ls += wm[w][c] == -INFINITY ? 0.f : wsum[w][c] * exp2f_fast(wm[w][c] - mx);
+    }
+    const int cg = c / Tq;
+    const int64_t row = ((int64_t)b * Hq + hk * G + cg) * Tq + (c - cg * Tq);
+    if (n_chunks == 1) {
+      const float inv = ls > 0.f ? 1.f / ls : 0.f;
+      *reinterpret_cast<bf16x4 *>(O + row * D + 4 * ch) =
+          pack4(t[0] * inv, t[1] * inv, t[2] * inv, t[3] * inv);
+      if (ch == 0) LSE[row] = ls > 0.f ? (mx + __log2f(ls)) * kLn2 : -INFINITY;
+    } else {
+      const int64_t slot = row * n_chunks + chunk;
+      *reinterpret_cast<f32x4 *>(part_o + slot * D + 4 * ch) = t;
+      if (ch == 0) *reinterpret_cast<f32x2 *>(part_ml + slot * 2) = f32x2{mx, ls};
+    }
   }
 }
 
 // Merge the n_splits partials of every query row: M = max m over partials with l > 0,
 // O = sum o_s 2^(m_s - M) / sum l_s 2^(m_s - M), LSE = (M + log2 sum) ln 2; a row with no
 // visible key gets O = 0, LSE = -inf.  One 256-thread workgroup per row: thread t sums
-// float4 column t % (D/4) over the partials s = t / (D/4) (mod 256 / (D/4)).  With PF > 0
-// (rows with many partials) its first PF partial rows and its (m, l) pair are loaded
-// before anything waits, so the row takes one memory round trip; then the threads reduce
-// M and the weights (kept in LDS), and the partials are weighted (a partial without keys
-// holds zeros and weight 0) and the groups added in a fixed order, so the result does not
-// depend on timing (nor on PF).
-template <int D, int PF>
+// float4 column t % (D/4) over the partials s = t / (D/4) (mod 256 / (D/4)).  The threads
+// reduce M and the weights (kept in LDS), then the partials are weighted (a partial without
+// keys holds zeros and weight 0) and the groups added in a fixed order, so the result does
+// not depend on timing.
+template <int D>
 __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
     const float *__restrict__ part_o, const float *__restrict__ part_ml, bf16 *__restrict__ O,
     float *__restrict__ LSE, int rows, int n_splits) {
@@ -234,12 +278,6 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   const float *ml = part_ml + (int64_t)row * n_splits * 2;
   const int c = tid % C4, sg = tid / C4;
   const f32x4 *po = reinterpret_cast<const f32x4 *>(part_o + (int64_t)row * n_splits * D) + c;
-  f32x4 xs[PF > 0 ? PF : 1];
-#pragma unroll
-  for (int j = 0; j < PF; ++j) {
-    const int s = sg + j * SG;
-    xs[j] = s < n_splits ? po[(int64_t)s * C4] : f32x4{};
-  }
   const f32x2 v0 = tid < n_splits ? *reinterpret_cast<const f32x2 *>(ml + 2 * tid) : f32x2{0.f, 0.f};
   float M = v0[1] > 0.f ? v0[0] : -INFINITY;
   for (int s = tid + 256; s < n_splits; s += 256) {
@@ -264,15 +302,8 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   __syncthreads();  // wts and the sums are visible
   lsum = (red[4] + red[5]) + (red[6] + red[7]);
   f32x4 acc{};
-#pragma unroll
-  for (int j = 0; j < PF; ++j) {
-    const int s = sg + j * SG;
-    const float w = s < n_splits ? wts[s] : 0.f;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) acc[e] = w != 0.f ? __builtin_fmaf(xs[j][e], w, acc[e]) : acc[e];
-  }
 #pragma unroll 4
-  for (int s = sg + PF * SG; s < n_splits; s += SG) {
+  for (int s = sg; s < n_splits; s += SG) {
     const f32x4 x = po[(int64_t)s * C4];
     const float w = wts[s];
 #pragma unroll
@@ -292,64 +323,73 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   if (tid == 0) LSE[row] = lsum > 0.f ? (M + __log2f(lsum)) * kLn2 : -INFINITY;
 }
 
-// Keys per wave: enough waves to fill the device (about 2048), at least 128 keys per
-// wave (so the block prefetch has work to hide behind), a multiple of 32, and at most
-// kDecMaxSplits partials per query row.
-DecodeSplit decode_split(int B, int Hkv, int Lmax) {
+// Workgroups per unit and waves per workgroup.
+//  * Enough workgroups to put 128 KB of load stages on every CU (256 of them with four
+//    waves at D = 128, 512 at D = 64), at least one 32-key block per wave: more, smaller
+//    workgroups pay their start and the merge again (32 x 4096 keys, D 128: 90.7 us with
+//    256, 96.2 with 512, 100.0 with 1024; 1 x 16000 keys, 12 heads, D 64: 18.8 with 256,
+//    16.5 with 512).
+//  * Caches of up to 16 blocks (512 keys) run as one chunk, in one launch: 8.3 us at 512
+//    keys, D 128, against 9.3 for four chunks and their merge.
+//  * D = 128 with at most 4096 blocks in all runs two waves per workgroup, at most 256
+//    workgroups: a short call is bound by the start of its workgroups, and two waves merge
+//    sooner (1 x 16384 keys, 8 heads: 19.2 against 19.9 us; 4 x 2000, 2 heads: 9.4 against
+//    10.7).  Above that four waves keep more loads in flight (8 x 8000, 8 heads: 43.2
+//    against 44.6).
+DecodeSplit decode_split(int B, int Hkv, int Lmax, int D) {
   const int64_t units = (int64_t)B * Hkv;
-  const int64_t target_waves = 2048;
-  int64_t per = ((int64_t)Lmax * units + target_waves - 1) / target_waves;
-  per = ((per + kDecBlock - 1) / kDecBlock) * kDecBlock;
-  if (per < 128) per = 128;
-  int64_t waves_per_unit = ((int64_t)Lmax + per - 1) / per;
-  while ((waves_per_unit + kDecWaves - 1) / kDecWaves * kDecWaves > kDecMaxSplits) {
-    per *= 2;
-    waves_per_unit = ((int64_t)Lmax + per - 1) / per;
-  }
+  const int64_t blocks = ((int64_t)Lmax + kDecBlock - 1) / kDecBlock;
   DecodeSplit s;
-  s.wkeys = (int)per;
-  s.n_chunks = (int)((waves_per_unit + kDecWaves - 1) / kDecWaves);
-  s.n_splits = s.n_chunks * kDecWaves;
+  if (blocks <= 16) {
+    s.n_waves = 4;
+    s.n_chunks = 1;
+    return s;
+  }
+  s.n_waves = D == 128 && units * blocks <= 4096 ? 2 : 4;
+  const int64_t fill = D == 128 ? 256 : 512;
+  const int64_t most = (blocks + s.n_waves - 1) / s.n_waves;
+  int64_t n = (fill + units - 1) / units;
+  n = n > most ? most : n;
+  s.n_chunks = (int)(n > kDecMaxSplits ? kDecMaxSplits : n);
   return s;
+}
+
+template <int D, int NW>
+static hipError_t launch_decode(const void *q, const void *k_cache, const void *v_cache,
+                                const int *cache_seqlens, void *o, float *lse, float *part_o,
+                                float *part_ml, int B, int Hq, int Hkv, int Tq, int Lmax,
+                                int n_chunks, float scale_log2, hipStream_t stream) {
+  constexpr size_t lds = NW * DecShape<D>::WAVE_LDS * sizeof(bf16);
+  // the kernel's static arrays come on top of the dynamic stages
+  if (lds + 2 * NW * 32 * sizeof(float) > 65536) {
+    hipError_t e = allow_lds<fa_decode_bf16_kernel<D, NW>>(lds);
+    if (e != hipSuccess) return e;
+  }
+  const dim3 grid((unsigned)((int64_t)B * Hkv * n_chunks)), block(64 * NW);
+  fa_decode_bf16_kernel<D, NW><<<grid, block, lds, stream>>>(
+      (const bf16 *)q, (const bf16 *)k_cache, (const bf16 *)v_cache, cache_seqlens, (bf16 *)o,
+      lse, part_o, part_ml, B, Hq, Hkv, Tq, Lmax, n_chunks, scale_log2);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || n_chunks == 1) return e;
+  const int rows = B * Hq * Tq;
+  fa_decode_combine_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
+      part_o, part_ml, (bf16 *)o, lse, rows, n_chunks);
+  return hipGetLastError();
 }
 
 hipError_t launch_decode_bf16(const void *q, const void *k_cache, const void *v_cache,
                               const int *cache_seqlens, void *o, float *lse, float *workspace,
                               int B, int Hq, int Hkv, int Tq, int Lmax, int D, float scale,
                               hipStream_t stream) {
-  const DecodeSplit sp = decode_split(B, Hkv, Lmax);
-  const int rows = B * Hq * Tq;
+  const DecodeSplit sp = decode_split(B, Hkv, Lmax, D);
   float *part_o = workspace;
-  float *part_ml = workspace + (int64_t)rows * sp.n_splits * D;
-  const float sl2 = scale * kLog2e;
-  const dim3 grid((unsigned)((int64_t)B * Hkv * sp.n_chunks)), block(256);
-  const dim3 cgrid((unsigned)rows), cblock(256);
-  const bool prefetch = sp.n_splits >= kCombinePrefetchMin;
-  auto combine = [&](auto kern) {
-    kern<<<cgrid, cblock, 0, stream>>>(part_o, part_ml, (bf16 *)o, lse, rows, sp.n_splits);
+  float *part_ml = workspace + (int64_t)B * Hq * Tq * sp.n_chunks * D;
+  auto go = [&](auto launch) {
+    return launch(q, k_cache, v_cache, cache_seqlens, o, lse, part_o, part_ml, B, Hq, Hkv, Tq,
+                  Lmax, sp.n_chunks, scale * kLog2e, stream);
   };
-  if (D == 64) {
-    fa_decode_bf16_kernel<64><<<grid, block, 0, stream>>>(
-        (const bf16 *)q, (const bf16 *)k_cache, (const bf16 *)v_cache, cache_seqlens, part_o,
-        part_ml, B, Hq, Hkv, Tq, Lmax, sp.n_chunks, sp.wkeys, sl2);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (prefetch)
-      combine(fa_decode_combine_kernel<64, kCombinePrefetch>);
-    else
-      combine(fa_decode_combine_kernel<64, 0>);
-  } else {
-    fa_decode_bf16_kernel<128><<<grid, block, 0, stream>>>(
-        (const bf16 *)q, (const bf16 *)k_cache, (const bf16 *)v_cache, cache_seqlens, part_o,
-        part_ml, B, Hq, Hkv, Tq, Lmax, sp.n_chunks, sp.wkeys, sl2);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    if (prefetch)
-      combine(fa_decode_combine_kernel<128, kCombinePrefetch>);
-    else
-      combine(fa_decode_combine_kernel<128, 0>);
-  }
-  return hipGetLastError();
+  if (D == 64) return go(launch_decode<64, 4>);
+  return sp.n_waves == 2 ? go(launch_decode<128, 2>) : go(launch_decode<128, 4>);
 }
 
 }  // namespace ttfa

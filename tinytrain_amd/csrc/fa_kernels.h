@@ -40,11 +40,10 @@ hipError_t launch_bwd_varlen_bf16(const void *q, const void *k, const void *v, c
 // KV-cache decode: q/o [B, Hq, Tq, D], caches [B, Hkv, Lmax, D], lse [B, Hq, Tq],
 // cache_seqlens [B] int32 on the device; workspace of decode_workspace_floats() floats.
 struct DecodeSplit {
-  int wkeys;     // keys per wave (a multiple of 32)
-  int n_chunks;  // workgroups per (batch, KV head)
-  int n_splits;  // partials per query row (4 per workgroup)
+  int n_waves;   // waves per workgroup
+  int n_chunks;  // workgroups per (batch, KV head), one partial per query row each
 };
-DecodeSplit decode_split(int B, int Hkv, int Lmax);
+DecodeSplit decode_split(int B, int Hkv, int Lmax, int D);
 hipError_t launch_decode_bf16(const void *q, const void *k_cache, const void *v_cache,
                               const int *cache_seqlens, void *o, float *lse, float *workspace,
                               int B, int Hq, int Hkv, int Tq, int Lmax, int D, float scale,

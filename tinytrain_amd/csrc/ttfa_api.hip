@@ -204,8 +204,8 @@ int ttfa_varlen_bwd(const void *q, const void *k, const void *v, const void *o,
 
 long long ttfa_decode_workspace_bytes(int B, int Hq, int Hkv, int Tq, int max_seqlen, int D) {
   if (check_decode(B, Hq, Hkv, Tq, max_seqlen, D, TTFA_BF16, 1.f)) return -1;
-  const ttfa::DecodeSplit sp = ttfa::decode_split(B, Hkv, max_seqlen);
-  return (long long)B * Hq * Tq * sp.n_splits * (D + 2) * (long long)sizeof(float);
+  const ttfa::DecodeSplit sp = ttfa::decode_split(B, Hkv, max_seqlen, D);
+  return (long long)B * Hq * Tq * sp.n_chunks * (D + 2) * (long long)sizeof(float);
 }
 
 int ttfa_decode_fwd(const void *q, const void *k_cache, const void *v_cache,
