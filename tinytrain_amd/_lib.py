@@ -7,11 +7,16 @@ The library is loaded on first use.  If it is missing, every call raises
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import threading
 from pathlib import Path
 
+import torch
+
 _PKG = Path(__file__).resolve().parent
 LIB_PATH = _PKG / "libttfa.so"
+NATIVE_PATH = _PKG / "_ttfa_torch.so"
 
 TTFA_BF16 = 0
 TTFA_F32 = 1
@@ -40,6 +45,7 @@ class TTFAError(RuntimeError):
         self.code = code
 
 
+_TENSOR_TYPES = (torch.Tensor, torch.nn.Parameter)
 _lock = threading.Lock()
 _lib = None
 
@@ -91,6 +97,34 @@ def load() -> ctypes.CDLL:
                 raise LibraryNotBuilt(f"{LIB_PATH} has ABI {ver}, expected {ABI_VERSION}; rebuild it")
             _lib = lib
     return _lib
+
+
+def plain_cuda(t) -> bool:
+    """A real GPU tensor (not a subclass such as a fake tensor): worth asking native()."""
+    return type(t) in _TENSOR_TYPES and t.is_cuda
+
+
+_native = None
+
+
+def native():
+    """Load (once) and return the extension of the native eager path (csrc/torch_native.cpp).
+    It calls libttfa.so, whose ABI version is checked first."""
+    global _native
+    if _native is None:
+        load()
+        with _lock:
+            if _native is None:
+                if not NATIVE_PATH.exists():
+                    raise LibraryNotBuilt(f"{NATIVE_PATH} is missing: build it with "
+                                          "`python -m tinytrain_amd.build`")
+                name = f"{__package__}._ttfa_torch"
+                loader = importlib.machinery.ExtensionFileLoader(name, str(NATIVE_PATH))
+                spec = importlib.util.spec_from_file_location(name, NATIVE_PATH, loader=loader)
+                mod = importlib.util.module_from_spec(spec)
+                loader.exec_module(mod)
+                _native = mod
+    return _native
 
 
 def strerror(code: int) -> str:

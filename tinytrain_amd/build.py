@@ -1,8 +1,10 @@
-"""Build recipe for libttfa.so (gfx950 only), in-tree.
+"""Build recipe for libttfa.so (gfx950 only) and _ttfa_torch.so, in-tree.
 
 ``python -m tinytrain_amd.build`` compiles every ``csrc/*.hip`` translation unit with
-hipcc for ``--offload-arch=gfx950`` in parallel and links ``tinytrain_amd/libttfa.so``.
-hipcc cross-compiles, so this runs on a host without a GPU.
+hipcc for ``--offload-arch=gfx950`` in parallel and links ``tinytrain_amd/libttfa.so``;
+beside it ``csrc/torch_native.cpp`` (host code: torch's C++ API over the C ABI) becomes the
+Python extension ``tinytrain_amd/_ttfa_torch.so``, linked against libttfa.so.  hipcc
+cross-compiles, so this runs on a host without a GPU.
 """
 
 from __future__ import annotations
@@ -18,6 +20,7 @@ PKG = Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 INCLUDE = PKG.parent / "include"
 LIB = PKG / "libttfa.so"
+NATIVE = PKG / "_ttfa_torch.so"
 OBJ_DIR = PKG / "_build"
 
 ARCH = "gfx950"
@@ -54,6 +57,40 @@ def _compile(src: Path, extra: list[str]) -> Path:
     return obj
 
 
+def _compile_native() -> Path:
+    """csrc/torch_native.cpp: host C++ only, with the HIP runtime's types."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths
+
+    obj = OBJ_DIR / "torch_native.o"
+    rocm = Path(_hipcc()).resolve().parent.parent
+    includes = [*include_paths(), sysconfig.get_paths()["include"], str(rocm / "include")]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-Wall",
+           "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{INCLUDE}",
+           *[x for d in includes for x in ("-isystem", d)],
+           "-c", str(CSRC / "torch_native.cpp"), "-o", str(obj)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_native.cpp:\n{res.stdout}\n{res.stderr}")
+    if res.stderr.strip():
+        print(res.stderr, file=sys.stderr)
+    return obj
+
+
+def _link_native(obj: Path) -> None:
+    from torch.utils.cpp_extension import library_paths
+
+    tmp = NATIVE.with_suffix(".so.tmp")
+    cmd = ["g++", "-shared", str(obj), f"-L{PKG}", "-l:libttfa.so", "-Wl,-rpath,$ORIGIN",
+           *[f"-L{d}" for d in library_paths()], "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch",
+           "-ltorch_python", "-o", str(tmp)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"link of {NATIVE.name} failed:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, NATIVE)
+
+
 def _generate() -> None:
     """Rewrites generated sources whose generator output has changed: the D = 64 stage
     schedule of the dK/dV pass (csrc/gen_dkdv64_asm.py -> csrc/dkdv64_item.inc), and the
@@ -75,21 +112,24 @@ def _generate() -> None:
 
 
 def build(verbose: bool = False, extra_flags: list[str] | None = None) -> Path:
-    """Compile all sources and link libttfa.so; returns the library path."""
+    """Compile all sources, link libttfa.so and _ttfa_torch.so; returns libttfa.so's path."""
     _generate()
     OBJ_DIR.mkdir(exist_ok=True)
     srcs = sorted(CSRC.glob("*.hip"))
     extra = list(extra_flags or [])
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
+        native = ex.submit(_compile_native)
         objs = list(ex.map(lambda s: _compile(s, extra), srcs))
+        native_obj = native.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB)
+    _link_native(native_obj)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources")
+        print(f"built {LIB} from {len(srcs)} sources, and {NATIVE.name}")
     return LIB
 
 

@@ -76,3 +76,18 @@ def flash_attn_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
 def _(q, k_cache, v_cache, cache_seqlens):
     B, Hq, Tq, D = q.shape
     return torch.empty_like(q), q.new_empty((B, Hq, Tq), dtype=torch.float32)
+
+
+class _NativeFirst(type(flash_attn_decode)):
+    """The custom op, with plain eager calls taken by the native path (csrc/torch_native.cpp;
+    None: the op's).  torch.compile and the torch.library tools see the op itself."""
+
+    def __call__(self, q, k_cache, v_cache, cache_seqlens):
+        if _lib.plain_cuda(q):
+            out = _lib.native().flash_attn_decode(q, k_cache, v_cache, cache_seqlens)
+            if out is not None:
+                return out
+        return super().__call__(q, k_cache, v_cache, cache_seqlens)
+
+
+flash_attn_decode.__class__ = _NativeFirst

@@ -150,8 +150,18 @@ def _backward_fn(ctx, do, dM):
 flash_attn_fwd.register_autograd(_backward_fn, setup_context=_setup_context)
 
 
+# The public functions take plain eager calls on GPU tensors through the native path
+# (csrc/torch_native.cpp: the same checks, allocations, C ABI calls and gradients without the
+# Python layers of the custom ops; a forward and backward cost 175 us of host time through
+# the ops).  It answers None for everything else -- other tensors, modes, transforms, inputs
+# outside the contract -- and then the custom op runs, as it does under torch.compile.
+
 def flash_attn(q, k, v):
     """Causal attention on contiguous [B, H, T, D] / [B, H_kv, T, D]; returns o."""
+    if not torch.compiler.is_compiling() and _lib.plain_cuda(q):
+        o = _lib.native().flash_attn(q, k, v)
+        if o is not None:
+            return o
     o, _ = flash_attn_fwd(q, k, v)
     return o
 
@@ -267,5 +277,9 @@ def flash_attn_varlen(q, k, v, cu_seqlens, max_seqlen):
     """Causal attention over packed sequences: q [Hq, total, D], k/v [Hkv, total, D] bf16,
     cu_seqlens int32 [n_seq + 1] (device), every sequence attending only within itself;
     returns o [Hq, total, D]."""
+    if not torch.compiler.is_compiling() and _lib.plain_cuda(q):
+        o = _lib.native().flash_attn_varlen(q, k, v, cu_seqlens, int(max_seqlen))
+        if o is not None:
+            return o
     o, _ = flash_attn_varlen_fwd(q, k, v, cu_seqlens, int(max_seqlen))
     return o

@@ -171,5 +171,10 @@ qk_norm_rope_fwd.register_autograd(_backward_fn, setup_context=_setup_context)
 
 def qk_norm_rope(q_raw, k_raw, v_raw, wq, wk, cos, sin, eps: float = 1e-6):
     """(q, k, v) for ``flash_attn`` from the [B, T, H, D] projections; see module doc."""
+    if not torch.compiler.is_compiling() and _lib.plain_cuda(q_raw):
+        # the native path (csrc/torch_native.cpp) for plain eager calls; None: the custom op's
+        out = _lib.native().qk_norm_rope(q_raw, k_raw, v_raw, wq, wk, cos, sin, float(eps))
+        if out is not None:
+            return out
     q, k, v, _, _ = qk_norm_rope_fwd(q_raw, k_raw, v_raw, wq, wk, cos, sin, float(eps))
     return q, k, v
