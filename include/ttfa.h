@@ -35,7 +35,7 @@
 extern "C" {
 #endif
 
-#define TTFA_ABI_VERSION 6
+#define TTFA_ABI_VERSION 7
 
 enum ttfa_dtype { TTFA_BF16 = 0, TTFA_F32 = 1 };
 
@@ -218,6 +218,25 @@ int ttfa_qk_prologue_fwd(const void *q_raw, const void *k_raw, const void *v_raw
                          const void *sin, void *q, void *k, void *v, float *rstd_q,
                          float *rstd_k, int B, int T, int Hq, int Hkv, int D, float eps,
                          void *hip_stream);
+
+/*
+ * ttfa_qk_prologue_fwd / _bwd with the RoPE tables in either type: table_dtype TTFA_BF16
+ * (as above) or TTFA_F32, the [T, D] fp32 tables, which the kernels round to bf16 as they
+ * read them (the same values, bitwise, without a cast of the tables before the call).
+ */
+int ttfa_qk_prologue_fwd_tables(const void *q_raw, const void *k_raw, const void *v_raw,
+                                const float *q_norm_w, const float *k_norm_w, const void *cos,
+                                const void *sin, int table_dtype, void *q, void *k, void *v,
+                                float *rstd_q, float *rstd_k, int B, int T, int Hq, int Hkv,
+                                int D, float eps, void *hip_stream);
+
+int ttfa_qk_prologue_bwd_tables(const void *dq, const void *dk, const void *dv,
+                                const void *q_raw, const void *k_raw, const float *q_norm_w,
+                                const float *k_norm_w, const void *cos, const void *sin,
+                                int table_dtype, const float *rstd_q, const float *rstd_k,
+                                void *dq_raw, void *dk_raw, void *dv_raw, float *dq_norm_w,
+                                float *dk_norm_w, float *workspace, int B, int T, int Hq,
+                                int Hkv, int D, void *hip_stream);
 
 /*
  * Bytes of fp32 workspace ttfa_qk_prologue_bwd needs for the given shape (per-

@@ -76,6 +76,29 @@ def test_forward_matches_oracle(B, T, Hq, Hkv, D):
     assert got[0].shape == (B, Hq, T, D) and got[0].is_contiguous()
 
 
+@pytest.mark.parametrize("D", [64, 128])
+def test_table_types_give_the_same_bits(D):
+    """fp32 tables (rounded inside the kernels), bf16 tables and tables that have to be cast
+    first (fp64, strided, on the CPU) give the same outputs and gradients, bitwise."""
+    announce(f"qk prologue tables D={D}")
+    B, T, Hq, Hkv = 2, 37, 4, 2
+    q, k, v, wq, wk, cos, sin = _dev(*_inputs(B, T, Hq, Hkv, D))
+    gs = [torch.randn(B, h, T, D, device=q.device).to(torch.bfloat16) for h in (Hq, Hkv, Hkv)]
+
+    def run(c, s):
+        ins = [t.clone().requires_grad_() for t in (q, k, v, wq, wk)]
+        outs = qk_norm_rope_fwd(*ins, c, s, 1e-6)[:3]
+        return [*outs, *torch.autograd.grad(outs, ins, gs)]
+
+    want = run(cos, sin)
+    wide = torch.stack([cos, sin], dim=-1)
+    for c, s in ((cos.bfloat16(), sin.bfloat16()), (cos, sin.bfloat16()), (cos.double(), sin.double()),
+                 (wide[..., 0], wide[..., 1]), (cos.cpu(), sin.cpu()),
+                 (torch.cat([cos, cos])[:T + 3].contiguous(), torch.cat([sin, sin])[:T + 3].contiguous())):
+        for a, b in zip(run(c, s), want):
+            assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("B,T,Hq,Hkv,D", SHAPES)
 def test_backward_matches_fp64_gradients(B, T, Hq, Hkv, D):
     announce(f"qk prologue bwd B={B} T={T} Hq={Hq} Hkv={Hkv} D={D}")

@@ -181,6 +181,18 @@ def test_abi_rejects_null_and_misaligned(call, n):
 
 
 @needs_lib
+def test_table_dtype_is_checked():
+    lib = _lib.load()
+    shape = (1, 8, 4, 2, 64)
+    for dt in (-1, 2):
+        assert lib.ttfa_qk_prologue_fwd_tables(*P[:7], dt, *P[7:12], *shape, 1e-6,
+                                               None) == _lib.E_DTYPE
+        assert lib.ttfa_qk_prologue_bwd_tables(*P[:9], dt, *P[9:17], *shape, None) == _lib.E_DTYPE
+    assert lib.ttfa_qk_prologue_fwd_tables(*P[:5], P[5] + 4, P[6], _lib.TTFA_F32, *P[7:12], *shape,
+                                           1e-6, None) == _lib.E_ALIGN
+
+
+@needs_lib
 @pytest.mark.parametrize("eps", [-1e-6, 1.0, float("nan")])
 def test_abi_rejects_bad_eps(eps):
     assert _fwd(eps=eps) == _lib.E_EPS

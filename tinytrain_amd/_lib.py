@@ -20,7 +20,7 @@ NATIVE_PATH = _PKG / "_ttfa_torch.so"
 
 TTFA_BF16 = 0
 TTFA_F32 = 1
-ABI_VERSION = 6
+ABI_VERSION = 7
 
 # Negative status codes of include/ttfa.h.
 E_NULL, E_HEAD_DIM, E_GROUP, E_SEQ, E_ALIGN, E_DTYPE, E_SCALE, E_EPS, E_QROWS, E_SCRATCH = (
@@ -30,7 +30,7 @@ EXPORTED = ("ttfa_abi_version", "ttfa_strerror", "ttfa_fwd", "ttfa_bwd", "ttfa_b
             "ttfa_bwd_dkdv", "ttfa_varlen_fwd", "ttfa_varlen_bwd", "ttfa_decode_workspace_bytes",
             "ttfa_decode_fwd", "ttfa_qk_prologue_fwd",
             "ttfa_qk_prologue_workspace_bytes", "ttfa_qk_prologue_bwd", "ttfa_bwd_static",
-            "ttfa_d128_wide")
+            "ttfa_d128_wide", "ttfa_qk_prologue_fwd_tables", "ttfa_qk_prologue_bwd_tables")
 
 
 class LibraryNotBuilt(RuntimeError):
@@ -64,6 +64,8 @@ _SIGS = {
     "ttfa_qk_prologue_fwd": ([_vp] * 12 + [_i] * 5 + [_f, _vp], _i),
     "ttfa_qk_prologue_workspace_bytes": ([_i] * 5, ctypes.c_longlong),
     "ttfa_qk_prologue_bwd": ([_vp] * 17 + [_i] * 5 + [_vp], _i),
+    "ttfa_qk_prologue_fwd_tables": ([_vp] * 7 + [_i] + [_vp] * 5 + [_i] * 5 + [_f, _vp], _i),
+    "ttfa_qk_prologue_bwd_tables": ([_vp] * 9 + [_i] + [_vp] * 8 + [_i] * 5 + [_vp], _i),
     "ttfa_bwd_static": ([_vp] * 9 + [_i] * 6 + [_f, _vp], _i),
     "ttfa_d128_wide": ([_i] * 3 + [ctypes.POINTER(_i)] * 2, _i),
 }

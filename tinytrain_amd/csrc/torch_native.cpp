@@ -298,10 +298,24 @@ struct Prologue {
   }
 };
 
-// Rows 0..T-1 of a RoPE table in bf16 (the reference's cos.to(x.dtype)).
-Tensor table(const Tensor &t, int64_t T) {
-  return t.narrow(0, 0, T).to(at::kBFloat16).contiguous();
-}
+// Rows 0..T-1 of the RoPE tables: fp32 ones go to the kernels as they are (rounded to bf16
+// there, the reference's cos.to(x.dtype)); anything else is cast to bf16 first.
+struct Tables {
+  Tensor cos, sin;
+  int dtype;
+
+  Tables(const Tensor &c, const Tensor &s, int64_t T) {
+    auto direct = [](const Tensor &t) {
+      return t.scalar_type() == at::kFloat && t.is_contiguous() &&
+             ((uintptr_t)t.const_data_ptr() & 15) == 0;
+    };
+    auto cast = [&](const Tensor &t) { return t.narrow(0, 0, T).to(at::kBFloat16).contiguous(); };
+    const bool as_is = direct(c) && direct(s);
+    cos = as_is ? c : cast(c);
+    sin = as_is ? s : cast(s);
+    dtype = as_is ? TTFA_F32 : TTFA_BF16;
+  }
+};
 
 Tensor weight(const Tensor &w) { return w.to(at::kFloat).contiguous(); }
 
@@ -314,14 +328,15 @@ PrologueOut prologue_fwd(const Prologue &p, double eps) {
   const int64_t B = p.q.size(0), T = p.q.size(1), Hq = p.q.size(2), D = p.q.size(3);
   const int64_t Hkv = p.k.size(2);
   const c10::DeviceGuard on(p.q.device());
-  const Tensor cb = table(p.cos, T), sb = table(p.sin, T), wq = weight(p.wq), wk = weight(p.wk);
+  const Tables tab(p.cos, p.sin, T);
+  const Tensor wq = weight(p.wq), wk = weight(p.wk);
   PrologueOut r{at::empty({B, Hq, T, D}, p.q.options()), at::empty({B, Hkv, T, D}, p.q.options()),
                 at::empty({B, Hkv, T, D}, p.q.options()), f32(p.q, {B, T, Hq}),
                 f32(p.q, {B, T, Hkv})};
-  check(ttfa_qk_prologue_fwd(
+  check(ttfa_qk_prologue_fwd_tables(
       p.q.const_data_ptr(), p.k.const_data_ptr(), p.v.const_data_ptr(), wq.const_data_ptr<float>(),
-      wk.const_data_ptr<float>(), cb.const_data_ptr(), sb.const_data_ptr(), r.q.mutable_data_ptr(),
-      r.k.mutable_data_ptr(), r.v.mutable_data_ptr(), r.rq.mutable_data_ptr<float>(),
+      wk.const_data_ptr<float>(), tab.cos.const_data_ptr(), tab.sin.const_data_ptr(), tab.dtype,
+      r.q.mutable_data_ptr(), r.k.mutable_data_ptr(), r.v.mutable_data_ptr(), r.rq.mutable_data_ptr<float>(),
       r.rk.mutable_data_ptr<float>(), (int)B, (int)T, (int)Hq, (int)Hkv, (int)D, (float)eps,
       stream_of(p.q)));
   return r;
@@ -335,7 +350,8 @@ Grads5 prologue_bwd(const Tensor &gq, const Tensor &gk, const Tensor &gv, const 
   const int64_t B = p.q.size(0), T = p.q.size(1), Hq = p.q.size(2), D = p.q.size(3);
   const int64_t Hkv = p.k.size(2);
   const c10::DeviceGuard on(p.q.device());
-  const Tensor cb = table(p.cos, T), sb = table(p.sin, T), wq = weight(p.wq), wk = weight(p.wk);
+  const Tables tab(p.cos, p.sin, T);
+  const Tensor wq = weight(p.wq), wk = weight(p.wk);
   const Tensor dq = gq.contiguous(), dk = gk.contiguous(), dv = gv.contiguous();
   Tensor dq_raw = same(p.q), dk_raw = same(p.k), dv_raw = same(p.k);
   Tensor dwq = f32(p.q, {D}), dwk = f32(p.q, {D});
@@ -343,10 +359,10 @@ Grads5 prologue_bwd(const Tensor &gq, const Tensor &gk, const Tensor &gv, const 
       ttfa_qk_prologue_workspace_bytes((int)B, (int)T, (int)Hq, (int)Hkv, (int)D);
   if (bytes < 0) check(TTFA_E_SEQ);
   Tensor ws = f32(p.q, {std::max<int64_t>(bytes / 4, 4)});
-  check(ttfa_qk_prologue_bwd(
+  check(ttfa_qk_prologue_bwd_tables(
       dq.const_data_ptr(), dk.const_data_ptr(), dv.const_data_ptr(), p.q.const_data_ptr(),
       p.k.const_data_ptr(), wq.const_data_ptr<float>(), wk.const_data_ptr<float>(),
-      cb.const_data_ptr(), sb.const_data_ptr(), rq.const_data_ptr<float>(),
+      tab.cos.const_data_ptr(), tab.sin.const_data_ptr(), tab.dtype, rq.const_data_ptr<float>(),
       rk.const_data_ptr<float>(), dq_raw.mutable_data_ptr(), dk_raw.mutable_data_ptr(),
       dv_raw.mutable_data_ptr(), dwq.mutable_data_ptr<float>(), dwk.mutable_data_ptr<float>(),
       ws.mutable_data_ptr<float>(), (int)B, (int)T, (int)Hq, (int)Hkv, (int)D, stream_of(p.q)));

@@ -66,9 +66,14 @@ def _check(q_raw, k_raw, v_raw, wq, wk, cos, sin):
 
 
 def _tables(cos, sin, T, device):
-    """Rows 0..T-1 of the RoPE tables in bf16 (apply_rope's cos.to(x.dtype))."""
+    """(cos, sin, C ABI dtype): rows 0..T-1 of the RoPE tables.  fp32 tables on the device go
+    to the kernels as they are (rounded to bf16 there, apply_rope's cos.to(x.dtype));
+    anything else is cast to bf16 first."""
+    if all(t.dtype == torch.float32 and t.device == device and t.is_contiguous()
+           and t.data_ptr() % 16 == 0 for t in (cos, sin)):
+        return cos, sin, _lib.TTFA_F32
     return (cos[:T].to(device=device, dtype=torch.bfloat16).contiguous(),
-            sin[:T].to(device=device, dtype=torch.bfloat16).contiguous())
+            sin[:T].to(device=device, dtype=torch.bfloat16).contiguous(), _lib.TTFA_BF16)
 
 
 def _stream(device):
@@ -78,7 +83,7 @@ def _stream(device):
 def _fwd(q_raw, k_raw, v_raw, wq, wk, cos, sin, eps):
     B, T, Hq, Hkv, D = _check(q_raw, k_raw, v_raw, wq, wk, cos, sin)
     dev = q_raw.device
-    cb, sb = _tables(cos, sin, T, dev)
+    ct, st, tab = _tables(cos, sin, T, dev)
     wq32, wk32 = wq.float().contiguous(), wk.float().contiguous()
     q = torch.empty((B, Hq, T, D), device=dev, dtype=torch.bfloat16)
     k = torch.empty((B, Hkv, T, D), device=dev, dtype=torch.bfloat16)
@@ -87,9 +92,9 @@ def _fwd(q_raw, k_raw, v_raw, wq, wk, cos, sin, eps):
     rk = torch.empty((B, T, Hkv), device=dev, dtype=torch.float32)
     lib = _lib.load()
     with torch.cuda.device(dev):
-        _lib.check(lib.ttfa_qk_prologue_fwd(
+        _lib.check(lib.ttfa_qk_prologue_fwd_tables(
             q_raw.data_ptr(), k_raw.data_ptr(), v_raw.data_ptr(), wq32.data_ptr(),
-            wk32.data_ptr(), cb.data_ptr(), sb.data_ptr(), q.data_ptr(), k.data_ptr(),
+            wk32.data_ptr(), ct.data_ptr(), st.data_ptr(), tab, q.data_ptr(), k.data_ptr(),
             v.data_ptr(), rq.data_ptr(), rk.data_ptr(), B, T, Hq, Hkv, D, float(eps),
             _stream(dev)))
     return q, k, v, rq, rk
@@ -99,7 +104,7 @@ def _bwd(dq, dk, dv, q_raw, k_raw, wq, wk, cos, sin, rq, rk):
     B, T, Hq, D = q_raw.shape
     Hkv = k_raw.shape[2]
     dev = q_raw.device
-    cb, sb = _tables(cos, sin, T, dev)
+    ct, st, tab = _tables(cos, sin, T, dev)
     wq32, wk32 = wq.float().contiguous(), wk.float().contiguous()
     dq, dk, dv = (t.to(torch.bfloat16).contiguous() for t in (dq, dk, dv))
     dq_raw = torch.empty_like(q_raw)
@@ -113,9 +118,9 @@ def _bwd(dq, dk, dv, q_raw, k_raw, wq, wk, cos, sin, rq, rk):
         _lib.check(_lib.E_SEQ)
     ws = torch.empty((max(nbytes // 4, 4),), device=dev, dtype=torch.float32)
     with torch.cuda.device(dev):
-        _lib.check(lib.ttfa_qk_prologue_bwd(
+        _lib.check(lib.ttfa_qk_prologue_bwd_tables(
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), q_raw.data_ptr(), k_raw.data_ptr(),
-            wq32.data_ptr(), wk32.data_ptr(), cb.data_ptr(), sb.data_ptr(), rq.data_ptr(),
+            wq32.data_ptr(), wk32.data_ptr(), ct.data_ptr(), st.data_ptr(), tab, rq.data_ptr(),
             rk.data_ptr(), dq_raw.data_ptr(), dk_raw.data_ptr(), dv_raw.data_ptr(),
             dwq.data_ptr(), dwk.data_ptr(), ws.data_ptr(), B, T, Hq, Hkv, D, _stream(dev)))
     return dq_raw, dk_raw, dv_raw, dwq.to(wq.dtype), dwk.to(wk.dtype)
