@@ -93,6 +93,23 @@ int ttfa_bwd(const void *q, const void *k, const void *v, const void *o,
              float scale, void *hip_stream);
 
 /*
+ * ttfa_bwd with a larger workspace: ttfa_bwd_workspace_bytes(...) bytes (-1 for an invalid
+ * shape), 16-byte aligned, overwritten.  Where one workgroup per 128 keys of a KV head
+ * would leave most of the device idle (few KV heads and a small batch), the dK/dV pass
+ * deals each key tile's work to several workgroups, whose fp32 partial sums in the
+ * workspace a further launch adds in a fixed order: still no atomics, bitwise
+ * reproducible, but rounded in another order than ttfa_bwd.  For every other shape it is
+ * ttfa_bwd.  A single sequence (B = 1) is split only at D = 128 and T > 1792, so that it
+ * keeps the bits of ttfa_varlen_bwd below.
+ */
+long long ttfa_bwd_workspace_bytes(int B, int Hq, int Hkv, int T, int D, int dtype);
+
+int ttfa_bwd_ws(const void *q, const void *k, const void *v, const void *o,
+                const void *dout, const float *lse, float *workspace, void *dq, void *dk,
+                void *dv, int B, int Hq, int Hkv, int T, int D, int dtype, float scale,
+                void *hip_stream);
+
+/*
  * ttfa_bwd without the delta_ws argument, for callers that cannot allocate device memory
  * (code under HIP graph capture, tight serving loops, harnesses that forbid hipMalloc).
  * No counterpart in the reference.  Delta (rowsum(o * dout), B * Hq * T fp32 values) goes

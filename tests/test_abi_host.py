@@ -94,6 +94,13 @@ def _bwd(ptrs=None, **kw):
                                 a["scale"], None)
 
 
+def _bwd_ws(ptrs=None, **kw):
+    a = {**OK, **kw}
+    p = P[:10] if ptrs is None else ptrs
+    return _lib.load().ttfa_bwd_ws(*p, a["B"], a["Hq"], a["Hkv"], a["T"], a["D"], a["dtype"],
+                                   a["scale"], None)
+
+
 def _bwd_dq(ptrs=None, **kw):
     a = {**OK, **kw}
     p = P[:8] if ptrs is None else ptrs
@@ -129,14 +136,15 @@ CASES = [
 
 
 @needs_lib
-@pytest.mark.parametrize("entry", [_fwd, _bwd, _bwd_dq, _bwd_dkdv])
+@pytest.mark.parametrize("entry", [_fwd, _bwd, _bwd_ws, _bwd_dq, _bwd_dkdv])
 @pytest.mark.parametrize("kw, code", CASES)
 def test_argument_errors_return_codes(entry, kw, code):
     assert entry(**kw) == code
 
 
 @needs_lib
-@pytest.mark.parametrize("entry, n", [(_fwd, 5), (_bwd, 10), (_bwd_dq, 8), (_bwd_dkdv, 8)])
+@pytest.mark.parametrize("entry, n", [(_fwd, 5), (_bwd, 10), (_bwd_ws, 10), (_bwd_dq, 8),
+                                      (_bwd_dkdv, 8)])
 def test_null_and_misaligned_pointers(entry, n):
     for i in range(n):
         ptrs = list(P[:n])
@@ -144,6 +152,27 @@ def test_null_and_misaligned_pointers(entry, n):
         assert entry(ptrs=ptrs) == _lib.E_NULL
         ptrs[i] = P[i] + 8
         assert entry(ptrs=ptrs) == _lib.E_ALIGN
+
+
+@needs_lib
+def test_bwd_workspace_bytes():
+    """Delta rows alone where the dK/dV pass is not split, whole 128-key fp32 tiles of dK and
+    dV beside them where it is; invalid shapes give -1."""
+    lib = _lib.load()
+    for B, Hq, Hkv, T, D in [(16, 12, 12, 1024, 64), (32, 12, 4, 1024, 64), (4, 16, 8, 4096, 128),
+                             (1, 16, 8, 16384, 128), (32, 8, 2, 512, 128), (1, 8, 2, 512, 128),
+                             (1, 8, 2, 4500, 64), (3, 2, 2, 1, 64)]:
+        n = lib.ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, _lib.TTFA_BF16)
+        assert n == 4 * -(-B * Hq * T // 4) * 4, (B, Hq, Hkv, T, D)
+    for B, Hq, Hkv, T, D in [(2, 8, 2, 512, 128), (3, 8, 2, 333, 128), (1, 8, 2, 8000, 128),
+                             (4, 8, 2, 1000, 64), (2, 8, 1, 3000, 64)]:
+        n = lib.ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, _lib.TTFA_BF16)
+        part = n - 4 * -(-B * Hq * T // 4) * 4
+        slots = 512 if D == 64 else 256
+        assert part % (2 * 128 * D * 4 * B * Hkv) == 0 and 0 < part <= slots * 2 * 128 * D * 4
+        assert lib.ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, _lib.TTFA_F32) < n
+    assert lib.ttfa_bwd_workspace_bytes(2, 8, 3, 512, 128, _lib.TTFA_BF16) == -1
+    assert lib.ttfa_bwd_workspace_bytes(2, 8, 2, 0, 128, _lib.TTFA_BF16) == -1
 
 
 @needs_lib

@@ -247,6 +247,55 @@ def test_large_groups(B, H, H_kv, T, D):
         assert_close_abs(nm, a, b, TOL_LSE if nm == "lse" else TOL[torch.bfloat16])
 
 
+@pytest.mark.parametrize("B, H, H_kv, T, D, split", [
+    (2, 8, 2, 512, 128, True),     # G = 4: pieces cross query heads
+    (2, 4, 4, 640, 128, False),    # longest list 5 stages: nothing to save
+    (2, 4, 4, 768, 128, True),     # 6 stages against 2: the shortest list that is split
+    (3, 6, 2, 333, 128, True),     # G = 3, ragged T, uneven pieces
+    (2, 8, 1, 129, 128, True),     # MQA, one row past a tile, the last tile in one piece
+    (1, 4, 2, 1792, 128, False),   # one sequence keeps the packed entry point's bits ...
+    (1, 4, 2, 1793, 128, True),    # ... up to here
+    (2, 16, 2, 130, 64, True),     # D = 64: 16 stages against 2
+    (2, 8, 2, 500, 64, True),
+    (2, 4, 4, 1200, 64, True),     # 10 stages against 2
+    (1, 8, 1, 2000, 64, False),
+    (9, 2, 1, 1500, 64, True),     # 9 units: not a multiple of the XCDs
+])
+def test_split_dkdv_pass(B, H, H_kv, T, D, split):
+    """Shapes that leave the device idle deal a key tile's query stages to several workgroups
+    (ttfa_bwd_ws): dK and dV against the oracle, dQ bitwise that of the unsplit pass, every
+    element written, nothing read from the workspace before it is written, run to run equal."""
+    announce(f"split dkdv B={B} H={H} Hkv={H_kv} T={T} D={D}")
+    lib = _lib.load()
+    q, k, v, do = make_custom(B, H, H_kv, T, D, torch.bfloat16, seed=B + T, do_scale=1e-2)
+    want = reference_outputs(q, k, v, do, dtype=torch.float64)
+    q, k, v, do = (t.to(DEV) for t in (q, k, v, do))
+    nbytes = lib.ttfa_bwd_workspace_bytes(B, H, H_kv, T, D, _lib.TTFA_BF16)
+    assert (nbytes > 4 * (B * H * T + 3)) == split
+    o, M = _forward(q, k, v)
+    s, sc, nan = torch.cuda.current_stream().cuda_stream, 1.0 / math.sqrt(D), float("nan")
+
+    def call(entry, ws):
+        outs = [torch.full_like(t, nan) for t in (q, k, v)]
+        _lib.check(entry(*[t.data_ptr() for t in (q, k, v, o, do, M, ws, *outs)], B, H, H_kv, T, D,
+                         _lib.TTFA_BF16, sc, s))
+        torch.cuda.synchronize()
+        return outs
+
+    one = call(lib.ttfa_bwd, torch.full((B * H * T,), nan, device=DEV))
+    ws = torch.full((nbytes // 4,), nan, device=DEV)
+    got = call(lib.ttfa_bwd_ws, ws)
+    again = call(lib.ttfa_bwd_ws, ws)
+    assert torch.equal(got[0], one[0])
+    for name, a, b, c, w in zip(("dq", "dk", "dv"), got, again, one, want[2:]):
+        assert torch.equal(a, b)
+        assert split or torch.equal(a, c)
+        assert_close_abs(name, a, w, TOL[torch.bfloat16])
+        # Against the unsplit sums: the same products added in fp32 in another order, each
+        # rounded to bf16 once, so within one bf16 step (2^-8) plus the sums' own 2^-15.
+        assert ((a.float() - c.float()).norm() <= 2 ** -8 * c.float().norm()).item(), name
+
+
 def _poisoned_call(q, k, v, do):
     """Call the C ABI with NaN-filled outputs: every element must be overwritten."""
     lib = _lib.load()

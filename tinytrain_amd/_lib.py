@@ -30,7 +30,8 @@ EXPORTED = ("ttfa_abi_version", "ttfa_strerror", "ttfa_fwd", "ttfa_bwd", "ttfa_b
             "ttfa_bwd_dkdv", "ttfa_varlen_fwd", "ttfa_varlen_bwd", "ttfa_decode_workspace_bytes",
             "ttfa_decode_fwd", "ttfa_qk_prologue_fwd",
             "ttfa_qk_prologue_workspace_bytes", "ttfa_qk_prologue_bwd", "ttfa_bwd_static",
-            "ttfa_d128_wide", "ttfa_qk_prologue_fwd_tables", "ttfa_qk_prologue_bwd_tables")
+            "ttfa_d128_wide", "ttfa_qk_prologue_fwd_tables", "ttfa_qk_prologue_bwd_tables",
+            "ttfa_bwd_workspace_bytes", "ttfa_bwd_ws")
 
 
 class LibraryNotBuilt(RuntimeError):
@@ -55,6 +56,8 @@ _SIGS = {
     "ttfa_strerror": ([_i], ctypes.c_char_p),
     "ttfa_fwd": ([_vp] * 5 + [_i] * 6 + [_f, _vp], _i),
     "ttfa_bwd": ([_vp] * 10 + [_i] * 6 + [_f, _vp], _i),
+    "ttfa_bwd_workspace_bytes": ([_i] * 6, ctypes.c_longlong),
+    "ttfa_bwd_ws": ([_vp] * 10 + [_i] * 6 + [_f, _vp], _i),
     "ttfa_bwd_dq": ([_vp] * 8 + [_i] * 6 + [_f, _vp], _i),
     "ttfa_bwd_dkdv": ([_vp] * 8 + [_i] * 6 + [_f, _vp], _i),
     "ttfa_varlen_fwd": ([_vp] * 6 + [_i] * 7 + [_f, _vp], _i),

@@ -28,6 +28,53 @@ __device__ __forceinline__ uint32_t lds_addr(const void *p) {
   return (uint32_t)(uintptr_t)(const TTFA_LDS void *)p;
 }
 
+// Split dK/dV pass: the G * (n_ktiles - kt) stages of key tile kt are dealt to n =
+// ceil(count / stages) pieces, evenly; the pieces of a unit (one KV head of one batch) are
+// numbered key tile by key tile.
+struct DkvPiece {
+  int kt, n, it0, it1;  // key tile, its piece count, this piece's stages
+};
+
+__host__ __device__ __forceinline__ int dkv_pieces_of(int kt, int n_ktiles, int G, int stages) {
+  return (G * (n_ktiles - kt) + stages - 1) / stages;
+}
+
+__device__ __forceinline__ DkvPiece dkv_piece(int piece, int n_ktiles, int G, int stages) {
+  int kt = 0, n = dkv_pieces_of(0, n_ktiles, G, stages);
+  while (piece >= n) {  // the grid holds exactly the unit's pieces, so kt stays < n_ktiles
+    piece -= n;
+    n = dkv_pieces_of(++kt, n_ktiles, G, stages);
+  }
+  const int count = G * (n_ktiles - kt);
+  return {kt, n, (int)((int64_t)count * piece / n), (int)((int64_t)count * (piece + 1) / n)};
+}
+
+// fp32 partial sums of one piece: the four waves' accumulators as they lie in registers,
+// [wave][dK | dV][column block][a][lane] of 4 floats (register 4a + e of the block), so
+// stores and the reducing reads are whole 1 KB rows.
+template <int D>
+struct DkvPart {
+  static constexpr int DB = D / 32;
+  static constexpr int FLOATS = 4 * 2 * DB * 4 * 64 * 4;
+  static __device__ __forceinline__ int at(int wave, int which, int db, int a, int lane) {
+    return ((((wave * 2 + which) * DB + db) * 4 + a) * 64 + lane) * 4;
+  }
+};
+
+template <int D>
+__device__ __forceinline__ void store_part(const f32x16 (&dk)[D / 32], const f32x16 (&dv)[D / 32],
+                                           float *part, int wave, int lane) {
+#pragma unroll
+  for (int db = 0; db < D / 32; ++db)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      *reinterpret_cast<f32x4 *>(part + DkvPart<D>::at(wave, 0, db, a, lane)) =
+          f32x4{dk[db][4 * a], dk[db][4 * a + 1], dk[db][4 * a + 2], dk[db][4 * a + 3]};
+      *reinterpret_cast<f32x4 *>(part + DkvPart<D>::at(wave, 1, db, a, lane)) =
+          f32x4{dv[db][4 * a], dv[db][4 * a + 1], dv[db][4 * a + 2], dv[db][4 * a + 3]};
+    }
+}
+
 template <int D>
 __global__ void fa_bwd_dq_bf16_kernel(const bf16 *__restrict__ Q, const bf16 *__restrict__ K,
                                       const bf16 *__restrict__ V, const bf16 *__restrict__ O,
@@ -55,6 +102,24 @@ __global__ void fa_bwd_dkdv_varlen_bf16_kernel(
     const bf16 *__restrict__ dO, const float *__restrict__ LSE, const float *__restrict__ Delta,
     bf16 *__restrict__ dK, bf16 *__restrict__ dV, const int *__restrict__ cu_seqlens, int n_seq,
     int total, int max_seqlen, int Hq, int Hkv, float scale_log2, float scale);
+template <int D>
+__global__ void fa_bwd_dkdv_split_bf16_kernel(
+    const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
+    const bf16 *__restrict__ dO, const float *__restrict__ LSE, const float *__restrict__ Delta,
+    bf16 *__restrict__ dK, bf16 *__restrict__ dV, float *__restrict__ part, int n_units, int Hq,
+    int Hkv, int T, int stages, float scale_log2, float scale);
+template <>
+__global__ void fa_bwd_dkdv_split_bf16_kernel<64>(
+    const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
+    const bf16 *__restrict__ dO, const float *__restrict__ LSE, const float *__restrict__ Delta,
+    bf16 *__restrict__ dK, bf16 *__restrict__ dV, float *__restrict__ part, int n_units, int Hq,
+    int Hkv, int T, int stages, float scale_log2, float scale);
+template <>
+__global__ void fa_bwd_dkdv_split_bf16_kernel<128>(
+    const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
+    const bf16 *__restrict__ dO, const float *__restrict__ LSE, const float *__restrict__ Delta,
+    bf16 *__restrict__ dK, bf16 *__restrict__ dV, float *__restrict__ part, int n_units, int Hq,
+    int Hkv, int T, int stages, float scale_log2, float scale);
 template <>
 __global__ void fa_bwd_dkdv_bf16_kernel<64>(const bf16 *__restrict__ Q, const bf16 *__restrict__ K,
                                             const bf16 *__restrict__ V, const bf16 *__restrict__ dO,

@@ -327,6 +327,53 @@ __global__ __launch_bounds__(256, (D == 64 ? 3 : 2)) void fa_bwd_dq_varlen_bf16_
 // generated stage streams of fa_bwd_dkdv64.hip and fa_bwd_dkdv128.hip (explicit
 // specializations declared in fa_bwd.h); their launchers are below.
 
+// dK and dV of the key tiles that dkdv_split dealt to several pieces: one workgroup per
+// (32-key wave block, dK or dV, key tile, unit), its waves one 32-column block each.  Every
+// value is the sum of the pieces' partials in piece order, rounded once.  The loads are
+// independent, so a wave keeps many of the pieces in flight; spread over all CUs the pass
+// reads at most 33 MB, from L2 and the MALL.
+template <int D>
+__global__ __launch_bounds__(2 * D) void fa_bwd_dkdv_reduce_kernel(
+    const float *__restrict__ part, bf16 *__restrict__ dK, bf16 *__restrict__ dV, int n_units,
+    int G, int T, int stages, float scale) {
+  constexpr int CH = D / 8;
+  __shared__ __attribute__((aligned(16))) bf16 tile[32 * D];
+  const int n_ktiles = (T + 127) / 128;
+  const int which = blockIdx.x & 1, wave_k = (blockIdx.x >> 1) & 3, rest = blockIdx.x >> 3;
+  const int kt = rest / n_units, unit = rest - kt * n_units;
+  int first = 0;  // pieces of the unit before this key tile's
+  for (int t = 0; t < kt; ++t) first += dkv_pieces_of(t, n_ktiles, G, stages);
+  const int n = dkv_pieces_of(kt, n_ktiles, G, stages);
+  const int db = wave_id(), lane = threadIdx.x & 63, lq = lane & 31, lg = lane >> 5;
+  const int64_t stride = (int64_t)n_units * DkvPart<D>::FLOATS;
+  const float *src = part + ((int64_t)first * n_units + unit) * DkvPart<D>::FLOATS +
+                     DkvPart<D>::at(wave_k, which, db, 0, lane);
+  f32x4 acc[4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) acc[a] = *reinterpret_cast<const f32x4 *>(src + 256 * a);
+#pragma unroll 4
+  for (int p = 1; p < n; ++p)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) acc[a] += *reinterpret_cast<const f32x4 *>(src + p * stride + 256 * a);
+  const float mul = which == 0 ? scale : 1.f;
+#pragma unroll
+  for (int a = 0; a < 4; ++a) {
+    const int col = 32 * db + 8 * a + 4 * lg;
+    *reinterpret_cast<bf16x4 *>(tile + lq * D + (swz<D>(lq, col >> 3) << 3) + (col & 7)) =
+        pack4(acc[a][0] * mul, acc[a][1] * mul, acc[a][2] * mul, acc[a][3] * mul);
+  }
+  __syncthreads();
+  bf16 *out = (which == 0 ? dK : dV) + (int64_t)unit * T * D;
+  const int row0 = kt * 128 + wave_k * 32;
+#pragma unroll
+  for (int i = 0; i < 32 * CH / (2 * D); ++i) {
+    const int e = threadIdx.x + 2 * D * i, row = e / CH, ch = e % CH;
+    if (row0 + row < T)
+      *reinterpret_cast<u32x4 *>(out + (int64_t)(row0 + row) * D + ch * 8) =
+          *reinterpret_cast<const u32x4 *>(tile + row * D + (swz<D>(row, ch) << 3));
+  }
+}
+
 // 256-row tiles, 64 rows per wave (fa_bwd_dq128.hip): half the LDS and L2 bytes per
 // product, but half the workgroups and a longer prologue per workgroup, so only where its
 // pairs fill the 256 resident slots of an MI355X and carry at least 18 key stages each
@@ -386,6 +433,84 @@ static hipError_t launch_dkdv(const void *q, const void *k, const void *v, const
                                      (const bf16 *)dout, lse, delta, (bf16 *)dk, (bf16 *)dv, B,
                                      Hq, Hkv, T, scale * kLog2e, scale, (int)paired);
   return hipGetLastError();
+}
+
+// Stages per piece of the split dK/dV pass, or no split.  One workgroup per key tile takes
+// as long as its longest list, G * n_ktiles stages in a row (about 3.7 us each at D = 128),
+// however idle the device is.  The split takes the fewest stages per piece (at least 2)
+// whose pieces still run in one round of the resident workgroups (256 at D = 128, 512 at
+// D = 64), so the pass takes that many stages, plus the partials' way through memory and the
+// reducing launch.  Measured on MI355X, whole backward, one workgroup per key tile -> split
+// (B x Hq/Hkv x T):
+//   D = 128:  3x8/2x333 55 -> 33 us, 4x8/2x1000 129 -> 65, 2x8/2x2000 241 -> 103,
+//             16x8/2x512 78 -> 61, 2x16/8x1500 122 -> 107, 1x8/2x8000 939 -> 513
+//   D = 64:   4x8/2x1000 82.5 -> 47, 2x12/4x2000 127 -> 76, 8x12/4x512 41 -> 36
+// Around the chosen size the time is flat (4x8/2x1000 with 2 .. 8 stages: 64.6-67.2).  It has
+// to save more stages than the partials cost: about 4 at D = 128; at D = 64, where two
+// workgroups share a CU and an idle device already runs each of them faster, more than half
+// of the list (3x12/12x900, 8 -> 4 stages, was 40.3 -> 43.6, and 2x12/12x2000, 16 -> 8,
+// 77.1 -> 79.3).
+// A single sequence keeps the unsplit sums, the bits of the packed entry point, except at
+// D = 128 above T = 1792, where those differ by the 256-row kernels too.
+DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
+  const DkdvSplit none{0, 0, 0};
+  if (B == 1 && !(D == 128 && T > 1792)) return none;
+  const int n = (T + 127) / 128, G = Hq / Hkv;
+  const int64_t units = (int64_t)B * Hkv, slots = D == 64 ? 512 : 256;
+  const int64_t longest = (int64_t)G * n;
+  if (units > slots || longest > (1 << 24)) return none;
+  auto pays = [&](int64_t st) { return longest >= (D == 64 ? 2 * st + 2 : st + 4); };
+  auto pieces = [&](int64_t st) {
+    int64_t p = 0;
+    for (int kt = 0; kt < n; ++kt) p += dkv_pieces_of(kt, n, G, (int)st);
+    return p;
+  };
+  const int64_t total = units * G * ((int64_t)n * (n + 1) / 2);
+  int64_t st = (total + slots - 1) / slots, p = 0;
+  for (st = st < 2 ? 2 : st; pays(st); st += 1 + st / 32)
+    if ((p = pieces(st)) * units <= slots) break;
+  if (!pays(st)) return none;
+  DkdvSplit s{(int)st, (int)p, 0};
+  while (s.split_tiles < n && dkv_pieces_of(s.split_tiles, n, G, s.stages) > 1) ++s.split_tiles;
+  return s;
+}
+
+int64_t dkdv_part_floats(const DkdvSplit &s, int B, int Hkv, int D) {
+  return (int64_t)s.pieces * B * Hkv * (D == 64 ? DkvPart<64>::FLOATS : DkvPart<128>::FLOATS);
+}
+
+template <int D>
+static hipError_t launch_dkdv_split(const void *q, const void *k, const void *v, const void *dout,
+                                    const float *lse, const float *delta, void *dk, void *dv,
+                                    float *part, const DkdvSplit &s, int B, int Hq, int Hkv,
+                                    int T, float scale, hipStream_t stream) {
+  constexpr size_t lds = D == 64 ? kDkv64LdsBytes : kDkv128LdsBytes;
+  if (lds > 65536) {
+    hipError_t e = allow_lds<fa_bwd_dkdv_split_bf16_kernel<D>>(lds);
+    if (e != hipSuccess) return e;
+  }
+  const int units = B * Hkv;
+  auto kern = fa_bwd_dkdv_split_bf16_kernel<D>;
+  kern<<<dim3((unsigned)(s.pieces * units)), dim3(256), lds, stream>>>(
+      (const bf16 *)q, (const bf16 *)k, (const bf16 *)v, (const bf16 *)dout, lse, delta,
+      (bf16 *)dk, (bf16 *)dv, part, units, Hq, Hkv, T, s.stages, scale * kLog2e, scale);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  fa_bwd_dkdv_reduce_kernel<D><<<dim3((unsigned)(8 * s.split_tiles * units)), dim3(2 * D), 0,
+                                 stream>>>(part, (bf16 *)dk, (bf16 *)dv, units, Hq / Hkv, T,
+                                           s.stages, scale);
+  return hipGetLastError();
+}
+
+hipError_t launch_bwd_dkdv_split_bf16(const void *q, const void *k, const void *v,
+                                      const void *dout, const float *lse, const float *delta,
+                                      void *dk, void *dv, float *part, const DkdvSplit &s, int B,
+                                      int Hq, int Hkv, int T, int D, float scale,
+                                      hipStream_t stream) {
+  return D == 64 ? launch_dkdv_split<64>(q, k, v, dout, lse, delta, dk, dv, part, s, B, Hq, Hkv, T,
+                                         scale, stream)
+                 : launch_dkdv_split<128>(q, k, v, dout, lse, delta, dk, dv, part, s, B, Hq, Hkv,
+                                          T, scale, stream);
 }
 
 template <int D>

@@ -47,8 +47,14 @@ __device__ __forceinline__ void dkdv64_stage(f32x16 (&dk)[2], f32x16 (&dv)[2], c
 // accumulated over the whole group in registers (no atomics), with 128-row Q/dO stages
 // double-buffered through LDS and each stage's compute one hand-scheduled block per wave.  Ends with a
 // workgroup barrier, so the caller may reuse the LDS ring right away.
+//
+// PART: only the stages [it0, it0 + n_part) of the key tile's list (query head major, then
+// query tile), whose fp32 sums go to part (DkvPart layout) instead of dk and dv, unless it
+// is null (the list is whole).
+template <bool PART = false>
 __device__ __forceinline__ void dkdv_rows64(bf16 *lds, const DkvHead &hd, int kt, float scale_log2,
-                                            float scale) {
+                                            float scale, int it0 = 0, int n_part = 0,
+                                            float *part = nullptr) {
   constexpr int D = 64, BMQ = 128, CH = D / 8, LOADS = BMQ * CH / 256;
   constexpr int TILE_BYTES = BMQ * D * 2, STAGE_BYTES = 2 * TILE_BYTES + 2 * BMQ * 4;
   const int G = hd.G, T = hd.T;
@@ -76,13 +82,14 @@ __device__ __forceinline__ void dkdv_rows64(bf16 *lds, const DkvHead &hd, int kt
 
   const int n_qt = (T + BMQ - 1) / BMQ;
   const int per_g = n_qt - kt;  // stages kt..n_qt-1 of each query head (kt holds the diagonal)
-  const int n_items = G * per_g;
+  const int n_items = PART ? n_part : G * per_g;
   const float inv_scale = 1.f / scale;
   // Each thread carries one LSE (tid < 128) or Delta value of the next stage from its load
   // to its staging, so nothing waits on the load until after the current stage's compute.
   float fl = 0.f;
   const uint32_t row_bytes = (uint32_t)T * 4;  // LSE / Delta rows past T read as zero
-  int ld_g = 0, ld_qt = kt;
+  int ld_g = PART ? it0 / per_g : 0, ld_qt = kt + (PART ? it0 - ld_g * per_g : 0);
+  int qt = ld_qt;  // query tile of the current item
   const int wave_u = wave_id();
   // global -> LDS: thread element e = 256i + tid covers row e / CH, physical chunk e % CH
   uint32_t voff[LOADS];
@@ -155,7 +162,6 @@ __device__ __forceinline__ void dkdv_rows64(bf16 *lds, const DkvHead &hd, int kt
   }
   __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): K/V registers complete before the loop
   __syncthreads();
-  int qt = kt;  // query tile of the current item
   for (int it = 0; it < n_items; ++it) {
     if (it + 1 < n_items) load_item((it + 1) & 1);
     const uint32_t so = (it & 1) * STAGE_BYTES;
@@ -170,6 +176,10 @@ __device__ __forceinline__ void dkdv_rows64(bf16 *lds, const DkvHead &hd, int kt
     __syncthreads();
   }
 
+  if (PART && part) {
+    store_part<D>(dkacc, dvacc, part, wave_u, lane);
+    return;
+  }
   // The loop's last barrier freed the LDS ring: each wave stages its dK and dV tiles in
   // its own two 32*D slices of it for row-contiguous stores.
   store_rows<D>(dkacc, scale, lds + wave * 64 * D, hd.dk, k0w, T, lane);
@@ -202,6 +212,29 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dkdv_bf16_kernel<64>(
     if (kt < 0) break;
     dkdv_rows64(smem, hd, kt, scale_log2, scale);
   }
+}
+
+// Batched, with every key tile's stages dealt to several workgroups (dkdv_split): workgroup
+// -> (piece of the unit, unit), piece-major, so the pieces of the longest key tiles start
+// first.  A key tile with one piece writes its dK and dV; the pieces of the others write
+// fp32 partial sums, which fa_bwd_dkdv_reduce_kernel adds in piece order.
+template <>
+__global__ __launch_bounds__(256, 2) void fa_bwd_dkdv_split_bf16_kernel<64>(
+    const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
+    const bf16 *__restrict__ dO, const float *__restrict__ LSE,
+    const float *__restrict__ Delta, bf16 *__restrict__ dK, bf16 *__restrict__ dV,
+    float *__restrict__ part, int n_units, int Hq, int Hkv, int T, int stages, float scale_log2,
+    float scale) {
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];
+  const int n_ktiles = (T + 127) / 128, G = Hq / Hkv;
+  const int piece = blockIdx.x / n_units, unit = blockIdx.x - piece * n_units;
+  const DkvPiece pc = dkv_piece(piece, n_ktiles, G, stages);
+  const int b = unit / Hkv, hk = unit - b * Hkv;
+  const int64_t hs = (int64_t)T * 64, kvb = unit * hs, q0 = (int64_t)b * Hq + hk * G;
+  const DkvHead hd{K + kvb, V + kvb, dK + kvb, dV + kvb, Q + q0 * hs, dO + q0 * hs,
+                   LSE + q0 * T, Delta + q0 * T, hs, T, G, T};
+  dkdv_rows64<true>(smem, hd, pc.kt, scale_log2, scale, pc.it0, pc.it1 - pc.it0,
+                   pc.n == 1 ? nullptr : part + (int64_t)blockIdx.x * DkvPart<64>::FLOATS);
 }
 
 // Packed variable-length sequences ([H, total, D] per tensor, sequence s at rows

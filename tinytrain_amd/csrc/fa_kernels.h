@@ -25,6 +25,22 @@ hipError_t launch_bwd_dkdv_bf16(const void *q, const void *k, const void *v, con
                                 int B, int Hq, int Hkv, int T, int D, float scale,
                                 hipStream_t stream);
 
+// How the dK/dV pass of a batched bf16 shape is split over workgroups (stages == 0: it is
+// not, one workgroup per key tile), and its launch with the fp32 partials of
+// dkdv_part_floats() floats.
+struct DkdvSplit {
+  int stages;       // 128-row stages per piece, at most
+  int pieces;       // pieces per (batch, KV head)
+  int split_tiles;  // key tiles 0 .. split_tiles - 1 have several pieces
+};
+DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D);
+int64_t dkdv_part_floats(const DkdvSplit &s, int B, int Hkv, int D);
+hipError_t launch_bwd_dkdv_split_bf16(const void *q, const void *k, const void *v,
+                                      const void *dout, const float *lse, const float *delta,
+                                      void *dk, void *dv, float *part, const DkdvSplit &s, int B,
+                                      int Hq, int Hkv, int T, int D, float scale,
+                                      hipStream_t stream);
+
 // Packed variable-length sequences, bf16: q/o [Hq, total, D], k/v [Hkv, total, D],
 // lse/delta [Hq, total]; cu_seqlens [n_seq + 1] int32 on the device.
 hipError_t launch_fwd_varlen_bf16(const void *q, const void *k, const void *v, void *o,

@@ -147,13 +147,15 @@ Grads3 attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
   RECORD_FUNCTION("tinytrain::flash_attn_bwd", c10::ArrayRef<const c10::IValue>());
   const c10::DeviceGuard on(q.device());
   const Tensor g = dout.contiguous();
-  Tensor delta = f32(q, {q.size(0), q.size(1), q.size(2)});
+  const int B = (int)q.size(0), Hq = (int)q.size(1), Hkv = (int)k.size(1), T = (int)q.size(2),
+            D = (int)q.size(3), dt = dtype_of(q);
+  const long long bytes = ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, dt);
+  Tensor ws = f32(q, {std::max<int64_t>(bytes / 4, 1)});
   Tensor dq = same(q), dk = same(k), dv = same(v);
-  check(ttfa_bwd(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(), o.const_data_ptr(),
-                 g.const_data_ptr(), M.const_data_ptr<float>(), delta.mutable_data_ptr<float>(),
-                 dq.mutable_data_ptr(), dk.mutable_data_ptr(), dv.mutable_data_ptr(),
-                 (int)q.size(0), (int)q.size(1), (int)k.size(1), (int)q.size(2), (int)q.size(3),
-                 dtype_of(q), scale_of(q.size(3)), stream_of(q)));
+  check(ttfa_bwd_ws(q.const_data_ptr(), k.const_data_ptr(), v.const_data_ptr(),
+                    o.const_data_ptr(), g.const_data_ptr(), M.const_data_ptr<float>(),
+                    ws.mutable_data_ptr<float>(), dq.mutable_data_ptr(), dk.mutable_data_ptr(),
+                    dv.mutable_data_ptr(), B, Hq, Hkv, T, D, dt, scale_of(D), stream_of(q)));
   return {dq, dk, dv};
 }
 

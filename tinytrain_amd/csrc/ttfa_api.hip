@@ -96,6 +96,14 @@ int check_ptrs(const void *const *ptrs, int n) {
   return TTFA_OK;
 }
 
+// The workspace of ttfa_bwd_ws: Delta rows, padded to 16 bytes, then the dK/dV partials.
+int64_t delta_floats(int B, int Hq, int T) { return ((int64_t)B * Hq * T + 3) / 4 * 4; }
+
+int64_t part_floats(int B, int Hq, int Hkv, int T, int D, int dtype) {
+  if (dtype != TTFA_BF16) return 0;
+  return ttfa::dkdv_part_floats(ttfa::dkdv_split(B, Hq, Hkv, T, D), B, Hkv, D);
+}
+
 }  // namespace
 
 extern "C" {
@@ -238,6 +246,30 @@ int ttfa_bwd(const void *q, const void *k, const void *v, const void *o, const v
   if (rc) return rc;
   return ttfa_bwd_dkdv(q, k, v, dout, lse, delta_ws, dk, dv, B, Hq, Hkv, T, D, dtype, scale,
                        hip_stream);
+}
+
+long long ttfa_bwd_workspace_bytes(int B, int Hq, int Hkv, int T, int D, int dtype) {
+  if (check_common(B, Hq, Hkv, T, D, dtype, 1.f)) return -1;
+  return 4ll * (delta_floats(B, Hq, T) + part_floats(B, Hq, Hkv, T, D, dtype));
+}
+
+int ttfa_bwd_ws(const void *q, const void *k, const void *v, const void *o, const void *dout,
+                const float *lse, float *workspace, void *dq, void *dk, void *dv, int B, int Hq,
+                int Hkv, int T, int D, int dtype, float scale, void *hip_stream) {
+  int rc = check_common(B, Hq, Hkv, T, D, dtype, scale);
+  if (rc) return rc;
+  const void *ptrs[] = {q, k, v, o, dout, lse, workspace, dq, dk, dv};
+  if ((rc = check_ptrs(ptrs, 10))) return rc;
+  const ttfa::DkdvSplit sp =
+      dtype == TTFA_BF16 ? ttfa::dkdv_split(B, Hq, Hkv, T, D) : ttfa::DkdvSplit{0, 0, 0};
+  if (sp.stages == 0)
+    return ttfa_bwd(q, k, v, o, dout, lse, workspace, dq, dk, dv, B, Hq, Hkv, T, D, dtype, scale,
+                    hip_stream);
+  rc = ttfa_bwd_dq(q, k, v, o, dout, lse, workspace, dq, B, Hq, Hkv, T, D, dtype, scale, hip_stream);
+  if (rc) return rc;
+  return static_cast<int>(ttfa::launch_bwd_dkdv_split_bf16(
+      q, k, v, dout, lse, workspace, dk, dv, workspace + delta_floats(B, Hq, T), sp, B, Hq, Hkv, T,
+      D, scale, static_cast<hipStream_t>(hip_stream)));
 }
 
 int ttfa_bwd_static(const void *q, const void *k, const void *v, const void *o,

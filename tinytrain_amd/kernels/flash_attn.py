@@ -94,15 +94,16 @@ def _backward(q, k, v, o, do, M):
         raise FlashAttnInputError("M must be the forward's fp32 [B, Hq, T] logsumexp")
     M = M.contiguous()
     lib = _lib.load()
-    delta = torch.empty((B * H, T), device=q.device, dtype=torch.float32)
+    nbytes = lib.ttfa_bwd_workspace_bytes(B, H, H_kv, T, D, _DTYPES[q.dtype])
+    ws = torch.empty((max(nbytes // 4, 1),), device=q.device, dtype=torch.float32)
     dq = torch.empty_like(q)
     dk = torch.empty_like(k)
     dv = torch.empty_like(v)
     with torch.cuda.device(q.device):
-        _lib.check(lib.ttfa_bwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
-                                do.data_ptr(), M.data_ptr(), delta.data_ptr(), dq.data_ptr(),
-                                dk.data_ptr(), dv.data_ptr(), B, H, H_kv, T, D,
-                                _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream_ptr(q.device)))
+        _lib.check(lib.ttfa_bwd_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(),
+                                   do.data_ptr(), M.data_ptr(), ws.data_ptr(), dq.data_ptr(),
+                                   dk.data_ptr(), dv.data_ptr(), B, H, H_kv, T, D,
+                                   _DTYPES[q.dtype], 1.0 / math.sqrt(D), _stream_ptr(q.device)))
     return dq, dk, dv
 
 
