@@ -296,6 +296,45 @@ def test_split_dkdv_pass(B, H, H_kv, T, D, split):
         assert ((a.float() - c.float()).norm() <= 2 ** -8 * c.float().norm()).item(), name
 
 
+@pytest.mark.parametrize("B, H, H_kv, T, D, split", [
+    (1, 8, 1, 96, 128, True),      # 48 items against 8
+    (2, 12, 4, 100, 128, False),   # 21 items: fewer than four rounds of the waves to save
+    (2, 8, 2, 113, 64, False),     # 32 items against 16
+    (2, 16, 2, 97, 64, True),      # 56 items against 16, ragged last block
+    (1, 6, 2, 345, 128, True),     # G = 3: pieces cross query heads
+    (2, 8, 2, 500, 128, True),
+])
+def test_split_fp32_backward(B, H, H_kv, T, D, split):
+    """fp32: a key block's items dealt to several workgroups, against the fp64 oracle and the
+    unsplit launch; every element written, nothing read before it is written, run to run
+    equal."""
+    announce(f"split fp32 backward B={B} H={H} Hkv={H_kv} T={T} D={D}")
+    lib, f32 = _lib.load(), _lib.TTFA_F32
+    q, k, v, do = make_custom(B, H, H_kv, T, D, torch.float32, seed=B + T, do_scale=1e-1)
+    q, k = (t * torch.rsqrt(t.pow(2).mean(-1, keepdim=True)) for t in (q, k))
+    want = reference_outputs(q, k, v, do, dtype=torch.float64)
+    q, k, v, do = (t.to(DEV) for t in (q, k, v, do))
+    nbytes = lib.ttfa_bwd_workspace_bytes(B, H, H_kv, T, D, f32)
+    assert (nbytes > 4 * (B * H * T + 3)) == split
+    o, M = _forward(q, k, v)
+    s, sc, nan = torch.cuda.current_stream().cuda_stream, 1.0 / math.sqrt(D), float("nan")
+
+    def call(entry, ws):
+        outs = [torch.full_like(t, nan) for t in (q, k, v)]
+        _lib.check(entry(*[t.data_ptr() for t in (q, k, v, o, do, M, ws, *outs)], B, H, H_kv, T, D,
+                         f32, sc, s))
+        torch.cuda.synchronize()
+        return outs
+
+    one = call(lib.ttfa_bwd, torch.full((B * H * T,), nan, device=DEV))
+    got = call(lib.ttfa_bwd_ws, torch.full((nbytes // 4,), nan, device=DEV))
+    again = call(lib.ttfa_bwd_ws, torch.full((nbytes // 4,), nan, device=DEV))
+    assert torch.equal(got[0], one[0])
+    for name, a, b, c, w in zip(("dq", "dk", "dv"), got, again, one, want[2:]):
+        assert torch.equal(a, b) and (split or torch.equal(a, c))
+        assert_close_abs(name, a, w, TOL[torch.float32])
+
+
 def _poisoned_call(q, k, v, do):
     """Call the C ABI with NaN-filled outputs: every element must be overwritten."""
     lib = _lib.load()

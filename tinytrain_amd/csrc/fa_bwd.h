@@ -35,18 +35,50 @@ struct DkvPiece {
   int kt, n, it0, it1;  // key tile, its piece count, this piece's stages
 };
 
-__host__ __device__ __forceinline__ int dkv_pieces_of(int kt, int n_ktiles, int G, int stages) {
-  return (G * (n_ktiles - kt) + stages - 1) / stages;
-}
+// Walks the key tiles of a unit in order with each one's piece count, without a division per
+// tile (a scalar division costs about 40 instructions, and a long sequence has hundreds of
+// tiles): spare is what the tile's pieces could hold beyond its list.
+struct DkvTiles {
+  int G, stages, kt = 0, n, spare;
+  __host__ __device__ __forceinline__ DkvTiles(int n_ktiles, int G_, int stages_)
+      : G(G_), stages(stages_) {
+    n = (G * n_ktiles + stages - 1) / stages;
+    spare = n * stages - G * n_ktiles;
+  }
+  __host__ __device__ __forceinline__ void next() {  // while kt < n_ktiles
+    ++kt;
+    spare += G;
+    while (spare >= stages) {
+      spare -= stages;
+      --n;
+    }
+  }
+};
 
 __device__ __forceinline__ DkvPiece dkv_piece(int piece, int n_ktiles, int G, int stages) {
-  int kt = 0, n = dkv_pieces_of(0, n_ktiles, G, stages);
-  while (piece >= n) {  // the grid holds exactly the unit's pieces, so kt stays < n_ktiles
-    piece -= n;
-    n = dkv_pieces_of(++kt, n_ktiles, G, stages);
+  if (stages >= G * n_ktiles) return {piece, 1, 0, G * (n_ktiles - piece)};
+  DkvTiles t(n_ktiles, G, stages);
+  while (piece >= t.n) {  // the grid holds exactly the unit's pieces, so kt stays < n_ktiles
+    piece -= t.n;
+    t.next();
   }
-  const int count = G * (n_ktiles - kt);
-  return {kt, n, (int)((int64_t)count * piece / n), (int)((int64_t)count * (piece + 1) / n)};
+  const int count = G * (n_ktiles - t.kt);
+  return {t.kt, t.n, (int)((int64_t)count * piece / t.n), (int)((int64_t)count * (piece + 1) / t.n)};
+}
+
+// Pieces of a unit before key tile kt, and kt's own count.
+struct DkvSlot {
+  int first, n;
+};
+
+__device__ __forceinline__ DkvSlot dkv_slot(int kt, int n_ktiles, int G, int stages) {
+  DkvTiles t(n_ktiles, G, stages);
+  int first = 0;
+  while (t.kt < kt) {
+    first += t.n;
+    t.next();
+  }
+  return {first, t.n};
 }
 
 // fp32 partial sums of one piece: the four waves' accumulators as they lie in registers,

@@ -341,18 +341,16 @@ __global__ __launch_bounds__(2 * D) void fa_bwd_dkdv_reduce_kernel(
   const int n_ktiles = (T + 127) / 128;
   const int which = blockIdx.x & 1, wave_k = (blockIdx.x >> 1) & 3, rest = blockIdx.x >> 3;
   const int kt = rest / n_units, unit = rest - kt * n_units;
-  int first = 0;  // pieces of the unit before this key tile's
-  for (int t = 0; t < kt; ++t) first += dkv_pieces_of(t, n_ktiles, G, stages);
-  const int n = dkv_pieces_of(kt, n_ktiles, G, stages);
+  const DkvSlot slot = dkv_slot(kt, n_ktiles, G, stages);
   const int db = wave_id(), lane = threadIdx.x & 63, lq = lane & 31, lg = lane >> 5;
   const int64_t stride = (int64_t)n_units * DkvPart<D>::FLOATS;
-  const float *src = part + ((int64_t)first * n_units + unit) * DkvPart<D>::FLOATS +
+  const float *src = part + ((int64_t)slot.first * n_units + unit) * DkvPart<D>::FLOATS +
                      DkvPart<D>::at(wave_k, which, db, 0, lane);
   f32x4 acc[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) acc[a] = *reinterpret_cast<const f32x4 *>(src + 256 * a);
 #pragma unroll 4
-  for (int p = 1; p < n; ++p)
+  for (int p = 1; p < slot.n; ++p)
 #pragma unroll
     for (int a = 0; a < 4; ++a) acc[a] += *reinterpret_cast<const f32x4 *>(src + p * stride + 256 * a);
   const float mul = which == 0 ? scale : 1.f;
@@ -460,9 +458,14 @@ DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
   const int64_t longest = (int64_t)G * n;
   if (units > slots || longest > (1 << 24)) return none;
   auto pays = [&](int64_t st) { return longest >= (D == 64 ? 2 * st + 2 : st + 4); };
+  int split_tiles = 0;
   auto pieces = [&](int64_t st) {
     int64_t p = 0;
-    for (int kt = 0; kt < n; ++kt) p += dkv_pieces_of(kt, n, G, (int)st);
+    DkvTiles t(n, G, (int)st);
+    for (split_tiles = 0; t.kt < n; t.next()) {
+      p += t.n;
+      split_tiles += t.n > 1;
+    }
     return p;
   };
   const int64_t total = units * G * ((int64_t)n * (n + 1) / 2);
@@ -470,9 +473,7 @@ DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
   for (st = st < 2 ? 2 : st; pays(st); st += 1 + st / 32)
     if ((p = pieces(st)) * units <= slots) break;
   if (!pays(st)) return none;
-  DkdvSplit s{(int)st, (int)p, 0};
-  while (s.split_tiles < n && dkv_pieces_of(s.split_tiles, n, G, s.stages) > 1) ++s.split_tiles;
-  return s;
+  return {(int)st, (int)p, split_tiles};
 }
 
 int64_t dkdv_part_floats(const DkdvSplit &s, int B, int Hkv, int D) {

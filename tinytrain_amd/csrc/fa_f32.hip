@@ -28,6 +28,7 @@
 // k-step r, which is exactly what the lane holds of a previous product: a product's
 // result feeds the next one as its B operand with no data movement; the other operand
 // is a column of a block ("column fragment").
+#include "fa_bwd.h"  // dkv_piece
 #include "fa_common.h"
 #include "fa_kernels.h"
 
@@ -37,9 +38,12 @@ namespace {
 
 constexpr int kF32Rows = 16;  // rows per block
 
-// Waves per workgroup: eight at D = 64 (two per SIMD, so one wave's dependent product
-// chain overlaps the other's), four at D = 128, whose operand registers do not leave
-// room for two waves per SIMD.
+// Waves per workgroup.  Forward: eight (two per SIMD, so one wave's dependent product chain
+// overlaps the other's; 239 registers at D = 128, where four waves and two workgroups per CU
+// took 25.8 us at 2x8/2x500 and 131 at 2x16/8x900 against 23.7 and 115: a workgroup's
+// serial chain halves and the second round balances the first).  Backward: eight at
+// D = 64, four at D = 128, whose operand registers do not leave room for two waves per SIMD.
+constexpr int kF32FwdWaves = 8;
 template <int D>
 constexpr int f32_waves() {
   return D == 64 ? 8 : 4;
@@ -181,14 +185,14 @@ __device__ __forceinline__ float *wave_tiles(float *lds, int wave) {
 }  // namespace
 
 template <int D>
-__global__ __launch_bounds__(64 * f32_waves<D>()) void fa_fwd_f32_kernel(const float *__restrict__ Q,
+__global__ __launch_bounds__(64 * kF32FwdWaves) void fa_fwd_f32_kernel(const float *__restrict__ Q,
                                                          const float *__restrict__ K,
                                                          const float *__restrict__ V,
                                                          float *__restrict__ O,
                                                          float *__restrict__ LSE, int Hq,
                                                          int Hkv, int T, int n_bh,
                                                          float scale) {
-  constexpr int NW = f32_waves<D>(), TPW = 2;
+  constexpr int NW = kF32FwdWaves, TPW = 2;
   __shared__ __attribute__((aligned(16))) float lds[NW * TPW * tile_floats<D>()];
   __shared__ float pm[NW][kF32Rows], pl[NW][kF32Rows];
   const int n_blk = (T + kF32Rows - 1) / kF32Rows;
@@ -394,8 +398,11 @@ constexpr int dkdv_tiles() {
 // dK and dV of key block kb of KV head bhk (LDS: NW * dkdv_tiles tiles).  OWN_DELTA:
 // form each query row's Delta from O and dO (the same sums, in the same order, as
 // dq_block) instead of reading it, so this pass need not wait for the dQ pass.
-template <int D, bool OWN_DELTA>
-__device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk, int kb) {
+// PART: only items [i0, i1), with the unscaled sums to part ([dK | dV] row-major tiles)
+// unless it is null.
+template <int D, bool OWN_DELTA, bool PART = false>
+__device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk, int kb, int i0 = 0,
+                                           int i1 = 0, float *part = nullptr) {
   constexpr int NW = f32_waves<D>(), TPW = dkdv_tiles<OWN_DELTA>();
   const int Hq = a.Hq, Hkv = a.Hkv, T = a.T;
   const float scale = a.scale;
@@ -409,7 +416,7 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
 
   // Items: (query head g of the group, query block qb >= kb), g-major; wave w takes the
   // items w, w + NW, ...
-  const int per_g = n_blk - kb, n_items = G * per_g;
+  const int per_g = n_blk - kb, n_items = PART ? i1 : G * per_g;
   struct Item {
     BlockRegs<D> q, dout;
     BlockRegs<OWN_DELTA ? D : 16> o;
@@ -430,7 +437,7 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
     }
   };
   Item nxt;
-  int i = wave;
+  int i = (PART ? i0 : 0) + wave;
   if (i < n_items) load_item(nxt, i);
 
   // K^T, V^T as B operands: row fragments of key k0 + n.
@@ -512,6 +519,12 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
       ov[e] += src[tile_floats<D>() + e];
     }
   }
+  if (PART && part) {
+    float *dst = part + mg.row * D + mg.c0;
+    store_chunk<M::CH>(dst, ok, 1.f);
+    store_chunk<M::CH>(dst + kF32Rows * D, ov, 1.f);
+    return;
+  }
   const int64_t o = ((int64_t)bhk * T + key) * D + mg.c0;
   store_chunk<M::CH>(a.dK + o, ok, scale);
   store_chunk<M::CH>(a.dV + o, ov, 1.f);
@@ -535,21 +548,60 @@ __global__ __launch_bounds__(64 * f32_waves<D>()) void fa_bwd_dkdv_f32_kernel(F3
   dkdv_block<D, false>(lds, a, bhk, kb);
 }
 
-// Both backward passes in one launch: the dK/dV workgroups form Delta themselves, so
-// they run beside the dQ workgroups instead of after them.  Workgroups go rank-major,
-// longest first in both roles: rank r holds the dK/dV blocks of key block r, then the
-// dQ blocks of query block n_blk - 1 - r.
+// Floats of one piece's partial: a 16-key tile of dK, then one of dV.
 template <int D>
-__global__ __launch_bounds__(64 * f32_waves<D>()) void fa_bwd_f32_kernel(F32Bwd a, int n_bh,
-                                                                          int n_bhk) {
+constexpr int kF32PartFloats = 2 * kF32Rows * D;
+
+// Both backward passes in one launch: the dK/dV workgroups form Delta themselves, so they
+// run beside the dQ workgroups instead of after them.  All dK/dV workgroups come first, the
+// longest key blocks leading, then the dQ blocks, longest first.  (Interleaved rank by rank,
+// the period of the workgroup ids put all dK/dV work of an XCD on the same few CUs: 161 us
+// against 82 at 2x12/4x700, D = 64, and 118 against 91 at 4x12/4x500.)
+//
+// The items of a key block may be dealt to several pieces (dkdv_split_f32): a key block with
+// one piece (all of them where items is the longest list) writes dK and dV; the others write
+// partial sums, which fa_bwd_f32_reduce_kernel adds in piece order.
+template <int D>
+__global__ __launch_bounds__(64 * f32_waves<D>()) void fa_bwd_f32_kernel(
+    F32Bwd a, float *__restrict__ part, int n_bh, int n_bhk, int n_pieces, int items) {
   __shared__ __attribute__((aligned(16))) float lds[f32_waves<D>() * 3 * tile_floats<D>()];
   const int n_blk = (a.T + kF32Rows - 1) / kF32Rows;
-  const int per_rank = n_bhk + n_bh;
-  const int rank = blockIdx.x / per_rank, x = blockIdx.x - rank * per_rank;
-  if (x < n_bhk)
-    dkdv_block<D, true>(lds, a, x, rank);
-  else
-    dq_block<D>(lds, a, x - n_bhk, n_blk - 1 - rank);
+  const int bid = blockIdx.x, n_dkdv = n_pieces * n_bhk;
+  if (bid < n_dkdv) {
+    const int piece = bid / n_bhk, unit = bid - piece * n_bhk;
+    const DkvPiece pc = dkv_piece(piece, n_blk, a.Hq / a.Hkv, items);
+    dkdv_block<D, true, true>(lds, a, unit, pc.kt, pc.it0, pc.it1,
+                              pc.n == 1 ? nullptr : part + (int64_t)bid * kF32PartFloats<D>);
+  } else {
+    const int rank = (bid - n_dkdv) / n_bh, bh = bid - n_dkdv - rank * n_bh;
+    dq_block<D>(lds, a, bh, n_blk - 1 - rank);
+  }
+}
+
+// dK and dV of the key blocks with several pieces: one workgroup per (key block, unit), a
+// float4 per thread and step, the pieces added in order.
+template <int D>
+__global__ __launch_bounds__(256) void fa_bwd_f32_reduce_kernel(const float *__restrict__ part,
+                                                                float *__restrict__ dK,
+                                                                float *__restrict__ dV,
+                                                                int n_bhk, int G, int T,
+                                                                int items, float scale) {
+  const int n_blk = (T + kF32Rows - 1) / kF32Rows;
+  const int kb = blockIdx.x / n_bhk, unit = blockIdx.x - kb * n_bhk;
+  const DkvSlot slot = dkv_slot(kb, n_blk, G, items);
+  const int64_t stride = (int64_t)n_bhk * kF32PartFloats<D>;
+  const float *src = part + ((int64_t)slot.first * n_bhk + unit) * kF32PartFloats<D>;
+#pragma unroll
+  for (int e = threadIdx.x * 4; e < kF32PartFloats<D>; e += 1024) {
+    f32x4 x = *reinterpret_cast<const f32x4 *>(src + e);
+#pragma unroll 4
+    for (int p = 1; p < slot.n; ++p) x += *reinterpret_cast<const f32x4 *>(src + p * stride + e);
+    const bool is_v = e >= kF32Rows * D;
+    const int r = is_v ? e - kF32Rows * D : e, key = kb * kF32Rows + r / D;
+    if (key < T)
+      *reinterpret_cast<f32x4 *>((is_v ? dV : dK) + ((int64_t)unit * T + key) * D + r % D) =
+          is_v ? x : x * scale;
+  }
 }
 
 static unsigned blocks_grid(int n_bh, int T) {
@@ -568,7 +620,7 @@ static F32Bwd bwd_args(const void *q, const void *k, const void *v, const void *
 
 hipError_t launch_fwd_f32(const void *q, const void *k, const void *v, void *o, float *lse,
                           int B, int Hq, int Hkv, int T, int D, float scale, hipStream_t stream) {
-  const dim3 grid(blocks_grid(B * Hq, T)), block = f32_block(D);
+  const dim3 grid(blocks_grid(B * Hq, T)), block = dim3(64 * kF32FwdWaves);
   if (D == 64)
     fa_fwd_f32_kernel<64><<<grid, block, 0, stream>>>((const float *)q, (const float *)k,
                                                       (const float *)v, (float *)o, lse, Hq,
@@ -607,17 +659,62 @@ hipError_t launch_bwd_dkdv_f32(const void *q, const void *k, const void *v, cons
   return hipGetLastError();
 }
 
+// Items per piece of a key block's list, or no split.  A key block of a KV head with many
+// query heads carries G * n_blk items (about 1.9 us per round of its waves), far more than
+// an even share of the launch for each of the 256 resident workgroups; pieces of one such
+// share bring the longest list down to it.  Measured, whole backward, one piece per key
+// block -> split: 2x8/2x500 D 128 109 -> 67 us, 1x8/2x1000 D 128 208 -> 114, 1x6/2x500 D 128
+// 83 -> 37, 4x6/2x130 D 128 28 -> 21, 1x8/2x1000 D 64 101 -> 60; half a share per piece was
+// slower (73, 117, 45, 21.5, 63).  It has to save four rounds of the waves, or the reducing
+// launch costs more (1x8/8x333 D 128, 3.25 rounds: 24.7 -> 27.6).
+DkdvSplit dkdv_split_f32(int B, int Hq, int Hkv, int T, int D) {
+  const DkdvSplit none{0, 0, 0};
+  const int n = (T + kF32Rows - 1) / kF32Rows, G = Hq / Hkv;
+  const int waves = D == 64 ? f32_waves<64>() : f32_waves<128>();
+  const int64_t units = (int64_t)B * Hkv, longest = (int64_t)G * n;
+  if (longest > (1 << 24) || units * longest > (1 << 28)) return none;
+  // all the work of the launch in dK/dV items: a dQ block pair is 3/4 of one
+  const int64_t total = units * G * ((int64_t)n * (n + 1) / 2) * 7 / 4;
+  int64_t items = (total / 256 + waves - 1) / waves * waves;
+  if (items < 2 * waves) items = 2 * waves;
+  if (longest - items < 4 * waves) return none;
+  DkdvSplit s{(int)items, 0, 0};
+  for (DkvTiles t(n, G, s.stages); t.kt < n; t.next()) {
+    s.pieces += t.n;
+    s.split_tiles += t.n > 1;
+  }
+  return s;
+}
+
+int64_t dkdv_part_floats_f32(const DkdvSplit &s, int B, int Hkv, int D) {
+  return (int64_t)s.pieces * B * Hkv * (D == 64 ? kF32PartFloats<64> : kF32PartFloats<128>);
+}
+
+template <int D>
+static hipError_t launch_bwd_f32_kernels(const F32Bwd &a, float *part, DkdvSplit s, int B,
+                                         hipStream_t stream) {
+  const int n_bh = B * a.Hq, n_bhk = B * a.Hkv, G = a.Hq / a.Hkv;
+  if (s.stages == 0) {  // one piece per key block
+    s.pieces = (a.T + kF32Rows - 1) / kF32Rows;
+    s.stages = G * s.pieces;
+  }
+  const unsigned grid = (unsigned)(s.pieces * n_bhk) + blocks_grid(n_bh, a.T);
+  fa_bwd_f32_kernel<D><<<dim3(grid), f32_block(D), 0, stream>>>(a, part, n_bh, n_bhk, s.pieces,
+                                                                s.stages);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || s.split_tiles == 0) return e;
+  fa_bwd_f32_reduce_kernel<D><<<dim3((unsigned)(s.split_tiles * n_bhk)), dim3(256), 0, stream>>>(
+      part, a.dK, a.dV, n_bhk, G, a.T, s.stages, a.scale);
+  return hipGetLastError();
+}
+
 hipError_t launch_bwd_f32(const void *q, const void *k, const void *v, const void *o,
                           const void *dout, const float *lse, float *delta, void *dq, void *dk,
-                          void *dv, int B, int Hq, int Hkv, int T, int D, float scale,
-                          hipStream_t stream) {
+                          void *dv, float *part, const DkdvSplit &s, int B, int Hq, int Hkv, int T,
+                          int D, float scale, hipStream_t stream) {
   const F32Bwd a = bwd_args(q, k, v, o, dout, lse, delta, dq, dk, dv, Hq, Hkv, T, scale);
-  const dim3 grid(blocks_grid(B * Hq + B * Hkv, T)), block = f32_block(D);
-  if (D == 64)
-    fa_bwd_f32_kernel<64><<<grid, block, 0, stream>>>(a, B * Hq, B * Hkv);
-  else
-    fa_bwd_f32_kernel<128><<<grid, block, 0, stream>>>(a, B * Hq, B * Hkv);
-  return hipGetLastError();
+  return D == 64 ? launch_bwd_f32_kernels<64>(a, part, s, B, stream)
+                 : launch_bwd_f32_kernels<128>(a, part, s, B, stream);
 }
 
 }  // namespace ttfa

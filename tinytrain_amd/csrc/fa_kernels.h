@@ -75,10 +75,14 @@ hipError_t launch_bwd_dkdv_f32(const void *q, const void *k, const void *v, cons
                                const float *lse, const float *delta, void *dk, void *dv,
                                int B, int Hq, int Hkv, int T, int D, float scale,
                                hipStream_t stream);
-// Both fp32 backward passes as one launch (same results, bitwise, as dq then dkdv).
+// Both fp32 backward passes as one launch.  Without a split (s.stages == 0; part unused) its
+// results are, bitwise, those of dq then dkdv; with one (`stages` = 16-row items here) a
+// second launch adds the partials of the split key blocks.
+DkdvSplit dkdv_split_f32(int B, int Hq, int Hkv, int T, int D);
+int64_t dkdv_part_floats_f32(const DkdvSplit &s, int B, int Hkv, int D);
 hipError_t launch_bwd_f32(const void *q, const void *k, const void *v, const void *o,
                           const void *dout, const float *lse, float *delta, void *dq, void *dk,
-                          void *dv, int B, int Hq, int Hkv, int T, int D, float scale,
-                          hipStream_t stream);
+                          void *dv, float *part, const DkdvSplit &s, int B, int Hq, int Hkv, int T,
+                          int D, float scale, hipStream_t stream);
 
 }  // namespace ttfa

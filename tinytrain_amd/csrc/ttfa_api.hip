@@ -99,9 +99,9 @@ int check_ptrs(const void *const *ptrs, int n) {
 // The workspace of ttfa_bwd_ws: Delta rows, padded to 16 bytes, then the dK/dV partials.
 int64_t delta_floats(int B, int Hq, int T) { return ((int64_t)B * Hq * T + 3) / 4 * 4; }
 
-int64_t part_floats(int B, int Hq, int Hkv, int T, int D, int dtype) {
-  if (dtype != TTFA_BF16) return 0;
-  return ttfa::dkdv_part_floats(ttfa::dkdv_split(B, Hq, Hkv, T, D), B, Hkv, D);
+ttfa::DkdvSplit split_of(int B, int Hq, int Hkv, int T, int D, int dtype) {
+  return dtype == TTFA_BF16 ? ttfa::dkdv_split(B, Hq, Hkv, T, D)
+                            : ttfa::dkdv_split_f32(B, Hq, Hkv, T, D);
 }
 
 }  // namespace
@@ -239,8 +239,9 @@ int ttfa_bwd(const void *q, const void *k, const void *v, const void *o, const v
   const void *ptrs[] = {q, k, v, o, dout, lse, delta_ws, dq, dk, dv};
   if ((rc = check_ptrs(ptrs, 10))) return rc;
   if (dtype == TTFA_F32)
-    return static_cast<int>(ttfa::launch_bwd_f32(q, k, v, o, dout, lse, delta_ws, dq, dk, dv, B,
-                                                 Hq, Hkv, T, D, scale,
+    return static_cast<int>(ttfa::launch_bwd_f32(q, k, v, o, dout, lse, delta_ws, dq, dk, dv,
+                                                 nullptr, ttfa::DkdvSplit{0, 0, 0}, B, Hq, Hkv, T,
+                                                 D, scale,
                                                  static_cast<hipStream_t>(hip_stream)));
   rc = ttfa_bwd_dq(q, k, v, o, dout, lse, delta_ws, dq, B, Hq, Hkv, T, D, dtype, scale, hip_stream);
   if (rc) return rc;
@@ -250,7 +251,10 @@ int ttfa_bwd(const void *q, const void *k, const void *v, const void *o, const v
 
 long long ttfa_bwd_workspace_bytes(int B, int Hq, int Hkv, int T, int D, int dtype) {
   if (check_common(B, Hq, Hkv, T, D, dtype, 1.f)) return -1;
-  return 4ll * (delta_floats(B, Hq, T) + part_floats(B, Hq, Hkv, T, D, dtype));
+  const ttfa::DkdvSplit sp = split_of(B, Hq, Hkv, T, D, dtype);
+  return 4ll * (delta_floats(B, Hq, T) + (dtype == TTFA_BF16
+                                              ? ttfa::dkdv_part_floats(sp, B, Hkv, D)
+                                              : ttfa::dkdv_part_floats_f32(sp, B, Hkv, D)));
 }
 
 int ttfa_bwd_ws(const void *q, const void *k, const void *v, const void *o, const void *dout,
@@ -260,16 +264,19 @@ int ttfa_bwd_ws(const void *q, const void *k, const void *v, const void *o, cons
   if (rc) return rc;
   const void *ptrs[] = {q, k, v, o, dout, lse, workspace, dq, dk, dv};
   if ((rc = check_ptrs(ptrs, 10))) return rc;
-  const ttfa::DkdvSplit sp =
-      dtype == TTFA_BF16 ? ttfa::dkdv_split(B, Hq, Hkv, T, D) : ttfa::DkdvSplit{0, 0, 0};
+  const ttfa::DkdvSplit sp = split_of(B, Hq, Hkv, T, D, dtype);
   if (sp.stages == 0)
     return ttfa_bwd(q, k, v, o, dout, lse, workspace, dq, dk, dv, B, Hq, Hkv, T, D, dtype, scale,
                     hip_stream);
+  float *part = workspace + delta_floats(B, Hq, T);
+  hipStream_t s = static_cast<hipStream_t>(hip_stream);
+  if (dtype == TTFA_F32)
+    return static_cast<int>(ttfa::launch_bwd_f32(q, k, v, o, dout, lse, workspace, dq, dk, dv, part,
+                                                 sp, B, Hq, Hkv, T, D, scale, s));
   rc = ttfa_bwd_dq(q, k, v, o, dout, lse, workspace, dq, B, Hq, Hkv, T, D, dtype, scale, hip_stream);
   if (rc) return rc;
-  return static_cast<int>(ttfa::launch_bwd_dkdv_split_bf16(
-      q, k, v, dout, lse, workspace, dk, dv, workspace + delta_floats(B, Hq, T), sp, B, Hq, Hkv, T,
-      D, scale, static_cast<hipStream_t>(hip_stream)));
+  return static_cast<int>(ttfa::launch_bwd_dkdv_split_bf16(q, k, v, dout, lse, workspace, dk, dv,
+                                                           part, sp, B, Hq, Hkv, T, D, scale, s));
 }
 
 int ttfa_bwd_static(const void *q, const void *k, const void *v, const void *o,
