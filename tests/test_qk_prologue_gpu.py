@@ -76,6 +76,18 @@ def test_forward_matches_oracle(B, T, Hq, Hkv, D):
     assert got[0].shape == (B, Hq, T, D) and got[0].is_contiguous()
 
 
+@pytest.mark.parametrize("B,T,Hq,Hkv,D", [
+    (3, 5, 3, 1, 64),      # a lane group's rows cross heads, positions and sequences
+    (7, 1, 1, 1, 128),     # every row another sequence
+    (1, 3, 2, 2, 64),      # fewer rows than one workgroup's groups
+    (2, 13, 5, 5, 128),
+    (1, 257, 1, 1, 64),    # one row past a backward workgroup, one head: a new table row each
+])
+def test_row_order_edges(B, T, Hq, Hkv, D):
+    test_forward_matches_oracle(B, T, Hq, Hkv, D)
+    test_backward_matches_fp64_gradients(B, T, Hq, Hkv, D)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_table_types_give_the_same_bits(D):
     """fp32 tables (rounded inside the kernels), bf16 tables and tables that have to be cast
