@@ -19,7 +19,10 @@
 // registers one block ahead of its use; at its turn the wave writes it to a
 // wave-private LDS tile and reads the MFMA operands back from there.  (Loading the
 // operands straight from global memory makes every load instruction touch 16 rows,
-// which saturates the per-CU load pipeline long before HBM or L2.)
+// which saturates the per-CU load pipeline long before HBM or L2.)  The LDS writes come
+// first and the next block's loads go into the same registers: loads issued before the
+// writes need a second set and a move per register, which cost the forward 21.4 -> 23.3 us
+// at 2x8/2x500 and 105.8 -> 114.7 at 2x16/8x900 (D = 128).
 //
 // MFMA 16x16x4 lane layout (lane = 16 j + n): A supplies A[n][j], B supplies B[j][n],
 // and register r of the result is D[4 j + r][n].  A contraction over D features uses
@@ -39,10 +42,12 @@ namespace {
 constexpr int kF32Rows = 16;  // rows per block
 
 // Waves per workgroup.  Forward: eight (two per SIMD, so one wave's dependent product chain
-// overlaps the other's; 239 registers at D = 128, where four waves and two workgroups per CU
+// overlaps the other's; 193 registers at D = 128, where four waves and two workgroups per CU
 // took 25.8 us at 2x8/2x500 and 131 at 2x16/8x900 against 23.7 and 115: a workgroup's
 // serial chain halves and the second round balances the first).  Backward: eight at
-// D = 64, four at D = 128, whose operand registers do not leave room for two waves per SIMD.
+// D = 64, four at D = 128, whose 340 operand registers do not leave room for two waves per
+// SIMD (with K and V re-read from LDS tiles eight fit, spilling 24: 67.2 us against 68.2 at
+// 2x8/2x500, but 27.5 against 21.4 at 4x6/2x130).
 constexpr int kF32FwdWaves = 8;
 template <int D>
 constexpr int f32_waves() {
@@ -228,13 +233,12 @@ __global__ __launch_bounds__(64 * kF32FwdWaves) void fa_fwd_f32_kernel(const flo
   for (int db = 0; db < D / 16; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (; kb <= qb; kb += NW) {
-    const Blk cur = nxt;
-    if (kb + NW <= qb) {  // in flight during this block
+    store_block<D>(tk, nxt.k, lane);
+    store_block<D>(tv, nxt.v, lane);
+    if (kb + NW <= qb) {  // in flight during this block's products
       load_block<D>(nxt.k, Kh, (kb + NW) * kF32Rows, last, lane);
       load_block<D>(nxt.v, Vh, (kb + NW) * kF32Rows, last, lane);
     }
-    store_block<D>(tk, cur.k, lane);
-    store_block<D>(tv, cur.v, lane);
     float kf[D / 4];
     read_rowfrag<D>(kf, tk, j, n);
     // S^T block: register r = score of key 16 kb + 4 j + r for query q0 + n.
@@ -349,13 +353,12 @@ __device__ __forceinline__ void dq_block(float *lds, const F32Bwd &a, int bh, in
   for (int db = 0; db < D / 16; ++db) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (; kb <= qb; kb += NW) {
-    const Blk cur = nxt;
-    if (kb + NW <= qb) {  // in flight during this block
+    store_block<D>(tk, nxt.k, lane);
+    store_block<D>(tv, nxt.v, lane);
+    if (kb + NW <= qb) {  // in flight during this block's products
       load_block<D>(nxt.k, Kh, (kb + NW) * kF32Rows, last, lane);
       load_block<D>(nxt.v, Vh, (kb + NW) * kF32Rows, last, lane);
     }
-    store_block<D>(tk, cur.k, lane);
-    store_block<D>(tv, cur.v, lane);
     float kf[D / 4], vf[D / 4];
     read_rowfrag<D>(kf, tk, j, n);
     read_rowfrag<D>(vf, tv, j, n);
@@ -390,12 +393,7 @@ __device__ __forceinline__ void dq_block(float *lds, const F32Bwd &a, int bh, in
   store_chunk<M::CH>(a.dQ + (hb + q) * D + mg.c0, out, scale);
 }
 
-template <bool OWN_DELTA>
-constexpr int dkdv_tiles() {
-  return OWN_DELTA ? 3 : 2;
-}
-
-// dK and dV of key block kb of KV head bhk (LDS: NW * dkdv_tiles tiles).  OWN_DELTA:
+// dK and dV of key block kb of KV head bhk (LDS: NW * 2 tiles).  OWN_DELTA:
 // form each query row's Delta from O and dO (the same sums, in the same order, as
 // dq_block) instead of reading it, so this pass need not wait for the dQ pass.
 // PART: only items [i0, i1), with the unscaled sums to part ([dK | dV] row-major tiles)
@@ -403,7 +401,7 @@ constexpr int dkdv_tiles() {
 template <int D, bool OWN_DELTA, bool PART = false>
 __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk, int kb, int i0 = 0,
                                            int i1 = 0, float *part = nullptr) {
-  constexpr int NW = f32_waves<D>(), TPW = dkdv_tiles<OWN_DELTA>();
+  constexpr int NW = f32_waves<D>(), TPW = 2;
   const int Hq = a.Hq, Hkv = a.Hkv, T = a.T;
   const float scale = a.scale;
   const int n_blk = (T + kF32Rows - 1) / kF32Rows;
@@ -412,7 +410,6 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
   const int b = bhk / Hkv, hk = bhk - b * Hkv;
   const int k0 = kb * kF32Rows, last = T - 1;
   float *tq = wave_tiles<D, TPW>(lds, wave), *tdo = tq + tile_floats<D>();
-  float *to = tdo + tile_floats<D>();  // OWN_DELTA only
 
   // Items: (query head g of the group, query block qb >= kb), g-major; wave w takes the
   // items w, w + NW, ...
@@ -428,7 +425,6 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
     const int q0 = qb * kF32Rows;
     load_block<D>(it.q, a.Q + qh * T * D, q0, last, lane);
     load_block<D>(it.dout, a.dO + qh * T * D, q0, last, lane);
-    if constexpr (OWN_DELTA) load_block<D>(it.o, a.O + qh * T * D, q0, last, lane);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int64_t x = qh * T + min(q0 + 4 * j + r, last);
@@ -436,9 +432,17 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
       if constexpr (!OWN_DELTA) it.delta[r] = a.Delta[x];
     }
   };
+  auto load_o = [&](Item &it, int i) {
+    const int g = i / per_g, qb = kb + (i - g * per_g);
+    const int64_t qh = (int64_t)b * Hq + hk * G + g;
+    if constexpr (OWN_DELTA) load_block<D>(it.o, a.O + qh * T * D, qb * kF32Rows, last, lane);
+  };
   Item nxt;
   int i = (PART ? i0 : 0) + wave;
-  if (i < n_items) load_item(nxt, i);
+  if (i < n_items) {
+    load_item(nxt, i);
+    load_o(nxt, i);
+  }
 
   // K^T, V^T as B operands: row fragments of key k0 + n.
   float kf[D / 4], vf[D / 4];
@@ -458,23 +462,19 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
   for (int db = 0; db < D / 16; ++db) dk[db] = dv[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   for (; i < n_items; i += NW) {
-    const Item cur = nxt;
-    if (i + NW < n_items) load_item(nxt, i + NW);  // in flight during this item
     const int g = i / per_g, qb = kb + (i - g * per_g), q0 = qb * kF32Rows;
-    store_block<D>(tq, cur.q, lane);
-    store_block<D>(tdo, cur.dout, lane);
+    float delta[4], lse[4];
+    store_block<D>(tdo, nxt.dout, lane);
     float qa[D / 4], doa[D / 4];
-    read_rowfrag<D>(qa, tq, j, n);
     read_rowfrag<D>(doa, tdo, j, n);
-    // S and dP: register r = query q0 + 4 j + r, key k0 + n.
-    const f32x4 s = dot_block<D>(qa, kf);
-    const f32x4 dp = dot_block<D>(doa, vf);
-    float delta[4];
     if constexpr (OWN_DELTA) {
-      // Delta of row q0 + n in every lane of column n, then row q0 + 4 j + r from lane 4 j + r.
+      // Delta of row q0 + n in every lane of column n, then row q0 + 4 j + r from lane 4 j + r
+      // (O passes through the Q tile, as in dq_block: a third tile per wave and O held with
+      // the other prefetches cost 69.1 us against 66.9 at 2x8/2x500 D = 128, 81.3 against 78.9
+      // at 2x12/4x700 D = 64).
       float oa[D / 4];
-      store_block<D>(to, cur.o, lane);
-      read_rowfrag<D>(oa, to, j, n);
+      store_block<D>(tq, nxt.o, lane);
+      read_rowfrag<D>(oa, tq, j, n);
       float d = 0.f;
 #pragma unroll
       for (int e = 0; e < D / 4; ++e) d = __builtin_fmaf(oa[e], doa[e], d);
@@ -483,16 +483,26 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
       for (int r = 0; r < 4; ++r) delta[r] = __shfl(d, 4 * j + r);
     } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) delta[r] = cur.delta[r];
+      for (int r = 0; r < 4; ++r) delta[r] = nxt.delta[r];
     }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) lse[r] = nxt.lse[r];
+    store_block<D>(tq, nxt.q, lane);
+    if (i + NW < n_items) load_item(nxt, i + NW);  // in flight during this item's products
+    read_rowfrag<D>(qa, tq, j, n);
+    // S and dP: register r = query q0 + 4 j + r, key k0 + n.
+    const f32x4 s = dot_block<D>(qa, kf);
+    const f32x4 dp = dot_block<D>(doa, vf);
     f32x4 p, ds;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int q = q0 + 4 * j + r;
       const bool keep = q < T && (qb != kb || n <= 4 * j + r);
-      p[r] = keep ? expf(s[r] * scale - cur.lse[r]) : 0.f;
+      p[r] = keep ? expf(s[r] * scale - lse[r]) : 0.f;
       ds[r] = p[r] * (dp[r] - delta[r]);
     }
+    // O of the next item only now: its registers were the fragments' until here.
+    if (i + NW < n_items) load_o(nxt, i + NW);
     float col[D / 4];
     read_colfrag<D>(col, tdo, j, n);
     accum_cols<D>(dv, col, p);   // dV^T += dO^T P
@@ -564,7 +574,7 @@ constexpr int kF32PartFloats = 2 * kF32Rows * D;
 template <int D>
 __global__ __launch_bounds__(64 * f32_waves<D>()) void fa_bwd_f32_kernel(
     F32Bwd a, float *__restrict__ part, int n_bh, int n_bhk, int n_pieces, int items) {
-  __shared__ __attribute__((aligned(16))) float lds[f32_waves<D>() * 3 * tile_floats<D>()];
+  __shared__ __attribute__((aligned(16))) float lds[f32_waves<D>() * 2 * tile_floats<D>()];
   const int n_blk = (a.T + kF32Rows - 1) / kF32Rows;
   const int bid = blockIdx.x, n_dkdv = n_pieces * n_bhk;
   if (bid < n_dkdv) {
