@@ -22,7 +22,7 @@ from tinytrain_amd.workloads import CONFIGS, make_custom, make_inputs
 from tinytrain_amd import _lib
 from tinytrain_amd.attention import Attention, RMSNorm, precompute_rope
 from tinytrain_amd.kernels.flash_attn import (_backward, _forward, flash_attn, flash_attn_bwd,
-                                              flash_attn_fwd)
+                                              flash_attn_fwd, flash_attn_varlen_fwd)
 
 pytestmark = pytest.mark.gpu
 
@@ -294,6 +294,43 @@ def test_split_dkdv_pass(B, H, H_kv, T, D, split):
         # Against the unsplit sums: the same products added in fp32 in another order, each
         # rounded to bf16 once, so within one bf16 step (2^-8) plus the sums' own 2^-15.
         assert ((a.float() - c.float()).norm() <= 2 ** -8 * c.float().norm()).item(), name
+
+
+@pytest.mark.parametrize("B, H, H_kv, T, D, split", [
+    (2, 4, 2, 193, 128, True),     # 4 key tiles, the last of one key
+    (2, 4, 2, 192, 128, False),
+    (3, 8, 2, 333, 128, True),     # the odd half of the first row tile sees one tile
+    (1, 4, 2, 1793, 128, False),   # one sequence keeps the packed entry point's bits
+    (2, 64, 8, 256, 128, True),    # 256 workgroups
+    (2, 65, 5, 256, 128, False),   # 260
+    (2, 4, 4, 321, 64, True),
+    (2, 4, 4, 320, 64, False),
+    (2, 12, 4, 700, 64, True),
+    (1, 4, 2, 2000, 64, False),
+])
+def test_split_forward(B, H, H_kv, T, D, split):
+    """Shapes that leave the device idle deal every row's key tiles to two halves of a
+    workgroup: O and LSE against the oracle, run to run equal, and against the packed entry
+    point, whose sums are never split."""
+    announce(f"split forward B={B} H={H} Hkv={H_kv} T={T} D={D}")
+    q, k, v, do = make_custom(B, H, H_kv, T, D, torch.bfloat16, seed=B + T, do_scale=1e-2)
+    want = reference_outputs(q, k, v, do, dtype=torch.float64)
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    o, M = _forward(q, k, v)
+    again = _forward(q, k, v)
+    cu = torch.arange(B + 1, dtype=torch.int32, device=DEV) * T
+    pack = lambda t: t.transpose(0, 1).reshape(t.shape[1], B * T, D).contiguous()  # noqa: E731
+    po, pM = flash_attn_varlen_fwd(pack(q), pack(k), pack(v), cu, T)
+    torch.cuda.synchronize()
+    po, pM = po.view(H, B, T, D).transpose(0, 1), pM.view(H, B, T).transpose(0, 1)
+    assert torch.equal(o, again[0]) and torch.equal(M, again[1])
+    assert_close_abs("O", o, want[0], TOL[torch.bfloat16])
+    assert_close_abs("LSE", M, want[1], TOL_LSE)
+    assert torch.equal(o, po) == (not split)
+    # The same fp32 terms added in another order: 2^-15 of the sums, in LSE absolute (natural
+    # log); O is rounded to bf16 once (2^-8) after its probabilities were, against another max.
+    assert (M - pM).abs().max().item() <= 2 ** -15
+    assert ((o.float() - po.float()).norm() <= 2 ** -8 * po.float().norm()).item()
 
 
 @pytest.mark.parametrize("B, H, H_kv, T, D, split", [

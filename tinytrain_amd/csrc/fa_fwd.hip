@@ -254,6 +254,121 @@ __device__ __forceinline__ void fwd_rows(bf16 (*lds)[2][FwdTile<D>::BN * D], con
   __syncthreads();  // the ring is free again for the caller
 }
 
+// fwd_rows with the key tiles of every row dealt to two halves of an eight-wave workgroup:
+// waves w and w + 4 own the same 32 rows, w takes the even tiles and w + 4 the odd ones, and
+// the two partials (unnormalised O, running max, sum) are merged through LDS.  A wave's pass
+// over its tiles is a serial chain (LDS reads -> scores -> softmax -> products), so where a
+// CU has a single workgroup half the chain is worth more than the merge costs.  A half whose
+// rows see none of its tiles contributes m = -inf, l = 0, O = 0.
+template <int D>
+__device__ __forceinline__ void fwd_rows_split(bf16 (*lds)[2][2][FwdTile<D>::BN * D],
+                                               float (*ml)[2][64], const FwdHead &hd, int qt,
+                                               float scale_log2) {
+  using P = FwdTile<D>;
+  constexpr int BM = P::BM, BN = P::BN, KK = P::KK, DB = P::DB, CH = P::CH, LOADS = P::LOADS;
+  const int T = hd.T;
+  const int wave = wave_id(), lane = threadIdx.x & 63;
+  const int half = wave >> 2, rw = wave & 3;  // scalar
+  const int lq = lane & 31, lg = lane >> 5;
+  const int q0 = qt * BM + rw * 32;  // first query row of this wave
+  const int qrow = q0 + lq;
+
+  const uint32_t head_bytes = (uint32_t)T * D * 2;
+  uint32_t voff[LOADS];
+#pragma unroll
+  for (int i = 0; i < LOADS; ++i) {
+    const int e = 256 * i + 64 * rw + lane, row = e / CH, pc = e % CH;
+    voff[i] = (uint32_t)(row * D + swz_l<D, kFwdLayout>(row, pc) * 8) * 2;
+  }
+  auto load_tile = [&](int j, int stage) {  // the half's four waves load its tile j
+    const int64_t t0 = (int64_t)j * BN * D;
+    const uint32_t left = head_bytes - (uint32_t)t0 * 2;
+    const auto rkj = make_rsrc(hd.k + t0, left), rvj = make_rsrc(hd.v + t0, left);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int e0 = 256 * i + 64 * rw;
+      buf_load16_lds(rkj, voff[i], &lds[stage][half][0][e0 * 8]);
+      buf_load16_lds(rvj, voff[i], &lds[stage][half][1][e0 * 8]);
+    }
+  };
+
+  const int n_kv = min((T + BN - 1) / BN, (qt + 1) * (BM / BN));
+  const int n_full = min((q0 + 1) / BN, T / BN);
+  const int n_vis = min(n_kv, (q0 + 31) / BN + 1);
+
+  // Q through stage 1 (its first half's K and V tiles), as in fwd_rows, loaded by all waves.
+  if (half < n_kv) load_tile(half, 0);
+  {
+    const uint32_t qbytes = head_bytes - (uint32_t)(qt * BM * D * 2);
+    const auto rqt = make_rsrc(hd.q + (int64_t)qt * BM * D, qbytes);
+    bf16 *Qs = &lds[1][0][0][0];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int e0 = 512 * i + 64 * wave, e = e0 + lane, row = e / CH, pc = e % CH;
+      buf_load16_lds(rqt, (uint32_t)(row * D + swz_l<D, kFwdLayout>(row, pc) * 8) * 2, Qs + e0 * 8);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  __syncthreads();
+  bf16x8 qf[KK];
+#pragma unroll
+  for (int kk = 0; kk < KK; ++kk)
+    qf[kk] = lds_read_row8<D, kFwdLayout>(&lds[1][0][0][0], rw * 32 + lq, 2 * kk + lg);
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): this wave's Q reads are complete
+  __syncthreads();                     // ... in every wave, before stage 1 is refilled
+
+  f32x16 oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; ++db) oacc[db] = f32x16{};
+  float m_t = -INFINITY;
+  float l_part = 0.f;
+  int stage = 0;
+  for (int r = 0; r < n_kv; r += 2, stage ^= 1) {  // the same count in both halves
+    const int j = r + half;
+    if (j + 2 < n_kv) load_tile(j + 2, stage ^ 1);
+    const bf16 *Kt = lds[stage][half][0];
+    const bf16 *Vt = lds[stage][half][1];
+    if (j < n_full)
+      fwd_tile<D, false>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, j * BN, qrow, T, lane);
+    else if (j < n_vis)
+      fwd_tile<D, true>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, j * BN, qrow, T, lane);
+    wait_vm_all();  // tile j+2 is in LDS before any wave passes the barrier
+    __syncthreads();
+  }
+
+  // The ring is free.  The odd half's partials go through stage 1, one 16-byte piece per
+  // lane and instruction; waves w and w + 4 hold the same elements in the same lanes.
+  const float l = xhalf_sum(l_part);
+  float *part = reinterpret_cast<float *>(&lds[1][0][0][0]) + rw * 32 * D + lane * 4;
+  if (half == 1) {
+#pragma unroll
+    for (int db = 0; db < DB; ++db)
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+        *reinterpret_cast<f32x4 *>(part + (4 * db + a) * 256) =
+            f32x4{oacc[db][4 * a], oacc[db][4 * a + 1], oacc[db][4 * a + 2], oacc[db][4 * a + 3]};
+    ml[rw][0][lane] = m_t;
+    ml[rw][1][lane] = l;
+  }
+  __syncthreads();
+  if (half == 1) return;
+  const float m1 = ml[rw][0][lane], l1 = ml[rw][1][lane], m = fmax2(m_t, m1);
+  const float a0 = exp2f_fast(m_t - m);  // the even half has tile 0, so its m is finite
+  const float a1 = m1 == -INFINITY ? 0.f : exp2f_fast(m1 - m);
+#pragma unroll
+  for (int db = 0; db < DB; ++db)
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const f32x4 x = *reinterpret_cast<const f32x4 *>(part + (4 * db + a) * 256);
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        oacc[db][4 * a + e] = __builtin_fmaf(x[e], a1, oacc[db][4 * a + e] * a0);
+    }
+  const float ls = __builtin_fmaf(l1, a1, l * a0);
+  store_rows<D>(oacc, 1.f / ls, &lds[0][0][0][0] + rw * 32 * D, hd.o, q0, T, lane);
+  if (qrow < T && lg == 0) hd.lse[qrow] = (m + __log2f(ls)) * kLn2;
+}
+
 template <int D>
 __global__ __launch_bounds__(256, 2) void fa_fwd_bf16_kernel(
     const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
@@ -284,6 +399,23 @@ __global__ __launch_bounds__(256, 2) void fa_fwd_bf16_kernel(
   } else {
     fwd_rows<D>(lds, hd, w.first, scale_log2, w1, wmax);
   }
+}
+
+// One row tile per eight-wave workgroup, longest first (fwd_rows_split).
+template <int D>
+__global__ __launch_bounds__(512, 2) void fa_fwd_split_bf16_kernel(
+    const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
+    bf16 *__restrict__ O, float *__restrict__ LSE, int B, int Hq, int Hkv, int T,
+    float scale_log2) {
+  using P = FwdTile<D>;
+  extern __shared__ __attribute__((aligned(16))) bf16 smem[];  // [stage][half][K|V]
+  __shared__ float ml[4][2][64];
+  const WorkPair w = single_item(blockIdx.x, (T + P::BM - 1) / P::BM, B, Hq, Hq / Hkv, false);
+  const int b = w.bh / Hq, h = w.bh - b * Hq;
+  const int64_t kvh = (int64_t)b * Hkv + h / (Hq / Hkv), hs = (int64_t)T * D;
+  const FwdHead hd{Q + w.bh * hs, K + kvh * hs, V + kvh * hs, O + w.bh * hs,
+                   LSE + (int64_t)w.bh * T, T};
+  fwd_rows_split<D>(reinterpret_cast<bf16 (*)[2][2][P::BN * D]>(smem), ml, hd, w.first, scale_log2);
 }
 
 // Packed variable-length sequences ([H, total, D] per tensor, sequence s at rows
@@ -341,6 +473,23 @@ bool fwd128_uses_wide(int B, int Hq, int T) {
   return n_wide >= 16 && (int64_t)sched_items(true, n_wide, B, Hq) >= kWideSlots;
 }
 
+// Key tiles dealt to two halves of the workgroup (fa_fwd_split_bf16_kernel) where at most one
+// workgroup per CU of an MI355X (kWideSlots) has work: the launch then lasts as long as the
+// longest row's chain of key tiles, and a second wave per SIMD hides part of it.  Forward,
+// four waves and eight: 1x8/2x2000 D128 39.4 -> 34.3 us, 4x8/2x1000 23.2 -> 21.0, 3x8/2x333
+// 11.4 -> 10.7; D64 2x8/2x2000 27.9 -> 24.3, 4x12/12x500 10.4 -> 9.5.  The merge is not repaid
+// on short rows (24x8/2x120 D128 7.5 -> 7.7, 16x8/2x200 9.8 -> 9.6; 16x4/4x300 D64 8.0 on both
+// sides), nor where the waves of several workgroups share the SIMDs anyway (32x8/2x512 D128
+// 28.9 -> 39.6, 16x12/12x1024 D64 35.8 -> 50.6).  A single sequence keeps the unsplit sums,
+// the bits of the packed entry point (1x8/2x2000 D128 would be 39.4 -> 34.3).
+// (Tried there and slower: 64- and 32-row workgroups, 18.9 -> 21.1 and 21.3 at 1x16/8x777 D128;
+// the next tile's scores computed among this tile's exponentials in one wave, 18.9 -> 21.7.)
+static bool fwd_uses_split(int B, int Hq, int T, int D) {
+  if (B == 1) return false;
+  const int64_t n_tiles = ((int64_t)T + FwdTile<64>::BM - 1) / FwdTile<64>::BM;
+  return T > (D == 64 ? 320 : 192) && n_tiles * B * Hq <= kWideSlots;
+}
+
 hipError_t launch_fwd_bf16(const void *q, const void *k, const void *v, void *o, float *lse,
                            int B, int Hq, int Hkv, int T, int D, float scale,
                            hipStream_t stream) {
@@ -357,6 +506,18 @@ hipError_t launch_fwd_bf16(const void *q, const void *k, const void *v, void *o,
         (const bf16 *)q, (const bf16 *)k, (const bf16 *)v, (bf16 *)o, lse, B, Hq, Hkv, T, sl2,
         (int)paired);
     return hipGetLastError();
+  }
+  if (fwd_uses_split(B, Hq, T, D)) {
+    auto split = [&](auto kern, hipError_t e, size_t lds) {
+      if (e != hipSuccess) return e;
+      kern<<<dim3((unsigned)(n_tiles * B * Hq)), dim3(512), lds, stream>>>(
+          (const bf16 *)q, (const bf16 *)k, (const bf16 *)v, (bf16 *)o, lse, B, Hq, Hkv, T, sl2);
+      return hipGetLastError();
+    };
+    constexpr size_t lds64 = 2 * 2 * 2 * 64 * 64 * 2, lds128 = 2 * lds64;
+    if (D == 64)
+      return split(fa_fwd_split_bf16_kernel<64>, allow_lds<fa_fwd_split_bf16_kernel<64>>(lds64), lds64);
+    return split(fa_fwd_split_bf16_kernel<128>, allow_lds<fa_fwd_split_bf16_kernel<128>>(lds128), lds128);
   }
   auto go = [&](auto kern, int slots) {
     const bool paired = use_pairs(n_tiles, B, Hq, slots);
