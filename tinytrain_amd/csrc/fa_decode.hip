@@ -336,6 +336,14 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
 //    sooner (1 x 16384 keys, 8 heads: 19.2 against 19.9 us; 4 x 2000, 2 heads: 9.4 against
 //    10.7).  Above that four waves keep more loads in flight (8 x 8000, 8 heads: 43.2
 //    against 44.6).
+//  * The workgroups of four waves stay within one round of those slots: a few above it ran as
+//    a second, nearly empty round (26 x 2 units, 4818 keys, D 128: 260 workgroups 29.0 us, 208
+//    24.2; 39 x 2, 6721: 312 63.4, 234 52.5; 47 x 2, 2649: 282 30.8, 188 25.3). At D = 64, where
+//    two workgroups share a CU, only where that leaves less than a tenth of the slots empty (14 x 12,
+//    13760: 672 81.5 us, 504 77.8; 16 x 12, 10267 keys of uneven caches: 576 52.1, 384 60.9).
+//    Up to one and a half rounds of D = 128 units of 2048 keys or more are halved, so that the
+//    second round is not one of whole units (36 x 8, 3352: 110.0 -> 102.1; 45 x 8, 5825: 149.5
+//    -> 140.7; but 33 x 8, 1043: 40.2 -> 41.4, and 53 x 8, 4946: 178.6 -> 196.4).
 DecodeSplit decode_split(int B, int Hkv, int Lmax, int D) {
   const int64_t units = (int64_t)B * Hkv;
   const int64_t blocks = ((int64_t)Lmax + kDecBlock - 1) / kDecBlock;
@@ -349,6 +357,11 @@ DecodeSplit decode_split(int B, int Hkv, int Lmax, int D) {
   const int64_t fill = D == 128 ? 256 : 512;
   const int64_t most = (blocks + s.n_waves - 1) / s.n_waves;
   int64_t n = (fill + units - 1) / units;
+  if (n > 1 && s.n_waves == 4 && (n - 1) * units >= (D == 128 ? 0 : fill - fill / 10)) {
+    if (n * units > fill) --n;  // one round of the slots
+  } else if (D == 128 && n == 1 && units > fill && 2 * units <= 3 * fill && blocks >= 64) {
+    n = 2;
+  }
   n = n > most ? most : n;
   s.n_chunks = (int)(n > kDecMaxSplits ? kDecMaxSplits : n);
   return s;
