@@ -83,7 +83,7 @@ class _NativeFirst(type(flash_attn_decode)):
     None: the op's).  torch.compile and the torch.library tools see the op itself."""
 
     def __call__(self, q, k_cache, v_cache, cache_seqlens):
-        if _lib.plain_cuda(q):
+        if not torch.compiler.is_compiling() and _lib.plain_cuda(q):
             out = _lib.native().flash_attn_decode(q, k_cache, v_cache, cache_seqlens)
             if out is not None:
                 return out
