@@ -82,6 +82,37 @@ def test_decode_splits_match_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
     assert_close_abs("lse", lse.cpu()[seen], want_lse[seen], TOL_LSE)
 
 
+@pytest.mark.parametrize("Hkv, L, D, lens, at", [
+    (2, 512, 128, [512, 20], [300, 3]),      # one chunk: a NaN in one wave of four, and in the
+    (2, 512, 64, [500, 32], [499, 0]),       # only wave with keys
+    (2, 2000, 128, [2000, 65], [1999, 64]),  # split, two waves per workgroup
+    (8, 9000, 128, [9000, 40], [5000, 39]),  # split, four waves
+    (2, 2000, 64, [1999, 40], [0, 7]),
+])
+@pytest.mark.parametrize("whole_block", [False, True])
+def test_decode_nan_keys_reach_the_result(Hkv, L, D, lens, at, whole_block):
+    """A NaN key makes O and LSE of exactly the rows that see it NaN, whichever workgroup and
+    wave reads it (alone among finite keys, or with its whole 32-key block); every other row
+    keeps its bits."""
+    announce(f"decode NaN Hkv={Hkv} L={L} D={D} lens={lens} at={at} block={whole_block}")
+    Tq = 2
+    q, k, v = (t.to(DEV) for t in _inputs(2, 2 * Hkv, Hkv, Tq, L, D, seed=5))
+    lens_t = torch.tensor(lens, dtype=torch.int32, device=DEV)
+    clean = flash_attn_decode(q, k, v, lens_t)
+    first = [a // 32 * 32 if whole_block else a for a in at]
+    for b in range(2):
+        k[b, 1, first[b]:at[b] + 1] = float("nan")
+    o, lse = flash_attn_decode(q, k, v, lens_t)
+    torch.cuda.synchronize()
+    pos = torch.tensor(lens)[:, None] + torch.arange(-Tq, 0)            # last key a row sees
+    bad = torch.zeros(2, 2 * Hkv, Tq, dtype=torch.bool)
+    bad[:, 2:4] = (torch.tensor(first)[:, None] <= pos)[:, None]        # KV head 1: q heads 2, 3
+    bad = bad.to(DEV)
+    assert torch.equal(torch.isnan(lse), bad)
+    assert torch.equal(torch.isnan(o), bad[..., None].expand_as(o))
+    assert torch.equal(o[~bad], clean[0][~bad]) and torch.equal(lse[~bad], clean[1][~bad])
+
+
 def test_decode_agrees_with_forward_kernel():
     announce("decode vs batched forward last rows")
     B, Hq, Hkv, T, D, Tq = 2, 8, 2, 700, 128, 2

@@ -212,7 +212,9 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
   // order.
   const float l = xhalf_sum(l_part);
   if (lg == 0) {
-    wm[wave][lq] = l > 0.f ? m_t : -INFINITY;  // a wave without visible keys weighs nothing
+    // A wave without visible keys (l exactly 0) weighs nothing.  A NaN sum is no empty one: its
+    // max may still be -inf (no score compares greater), and then the sum is relative to 0.
+    wm[wave][lq] = l == 0.f ? -INFINITY : m_t == -INFINITY ? 0.f : m_t;
     wsum[wave][lq] = l;
   }
   __syncthreads();
@@ -247,10 +249,10 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
     const int cg = c / Tq;
     const int64_t row = ((int64_t)b * Hq + hk * G + cg) * Tq + (c - cg * Tq);
     if (n_chunks == 1) {
-      const float inv = ls > 0.f ? 1.f / ls : 0.f;
+      const float inv = ls == 0.f ? 0.f : 1.f / ls;  // NaN sums reach O and LSE
       *reinterpret_cast<bf16x4 *>(O + row * D + 4 * ch) =
           pack4(t[0] * inv, t[1] * inv, t[2] * inv, t[3] * inv);
-      if (ch == 0) LSE[row] = ls > 0.f ? (mx + __log2f(ls)) * kLn2 : -INFINITY;
+      if (ch == 0) LSE[row] = ls == 0.f ? -INFINITY : (mx + __log2f(ls)) * kLn2;
     } else {
       const int64_t slot = row * n_chunks + chunk;
       *reinterpret_cast<f32x4 *>(part_o + slot * D + 4 * ch) = t;
@@ -259,9 +261,9 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
   }
 }
 
-// Merge the n_splits partials of every query row: M = max m over partials with l > 0,
+// Merge the n_splits partials of every query row: M = max m over partials with l != 0,
 // O = sum o_s 2^(m_s - M) / sum l_s 2^(m_s - M), LSE = (M + log2 sum) ln 2; a row with no
-// visible key gets O = 0, LSE = -inf.  One 256-thread workgroup per row: thread t sums
+// visible key (every l exactly 0) gets O = 0, LSE = -inf, and a NaN sum makes both NaN.  One 256-thread workgroup per row: thread t sums
 // float4 column t % (D/4) over the partials s = t / (D/4) (mod 256 / (D/4)).  The threads
 // reduce M and the weights (kept in LDS), then the partials are weighted (a partial without
 // keys holds zeros and weight 0) and the groups added in a fixed order, so the result does
@@ -279,10 +281,10 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   const int c = tid % C4, sg = tid / C4;
   const f32x4 *po = reinterpret_cast<const f32x4 *>(part_o + (int64_t)row * n_splits * D) + c;
   const f32x2 v0 = tid < n_splits ? *reinterpret_cast<const f32x2 *>(ml + 2 * tid) : f32x2{0.f, 0.f};
-  float M = v0[1] > 0.f ? v0[0] : -INFINITY;
+  float M = v0[1] != 0.f ? v0[0] : -INFINITY;
   for (int s = tid + 256; s < n_splits; s += 256) {
     const f32x2 v = *reinterpret_cast<const f32x2 *>(ml + 2 * s);
-    if (v[1] > 0.f) M = fmax2(M, v[0]);
+    if (v[1] != 0.f) M = fmax2(M, v[0]);
   }
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) M = fmax2(M, __shfl_xor(M, m));
@@ -292,9 +294,9 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   float lsum = 0.f;
   for (int s = tid; s < n_splits; s += 256) {
     const f32x2 v = s == tid ? v0 : *reinterpret_cast<const f32x2 *>(ml + 2 * s);
-    const float w = (v[1] > 0.f && M != -INFINITY) ? exp2f_fast(v[0] - M) : 0.f;
+    const float w = v[1] != 0.f ? exp2f_fast(v[0] - M) : 0.f;
     wts[s] = w;
-    lsum = __builtin_fmaf(v[1] > 0.f ? v[1] : 0.f, w, lsum);
+    lsum = __builtin_fmaf(v[1], w, lsum);
   }
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) lsum += __shfl_xor(lsum, m);
@@ -315,12 +317,12 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
     f32x4 t = accs[0][tid];
 #pragma unroll
     for (int g = 1; g < SG; ++g) t += accs[g][tid];
-    const float inv = lsum > 0.f ? 1.f / lsum : 0.f;
+    const float inv = lsum == 0.f ? 0.f : 1.f / lsum;
     bf16 *out = O + (int64_t)row * D + 4 * tid;
 #pragma unroll
     for (int e = 0; e < 4; ++e) out[e] = (bf16)(t[e] * inv);
   }
-  if (tid == 0) LSE[row] = lsum > 0.f ? (M + __log2f(lsum)) * kLn2 : -INFINITY;
+  if (tid == 0) LSE[row] = lsum == 0.f ? -INFINITY : (M + __log2f(lsum)) * kLn2;
 }
 
 // Workgroups per unit and waves per workgroup.
