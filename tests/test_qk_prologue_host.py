@@ -250,3 +250,23 @@ def test_input_errors_are_loud(bad, msg):
         q, k, v = q[..., :32], k[..., :32], v[..., :32]
     with pytest.raises(qp.QKPrologueInputError, match=msg):
         qp.qk_norm_rope(q, k, v, wq, wk, cos, sin)
+
+
+@pytest.mark.parametrize("i, change, msg", [
+    (0, lambda t: t[:, :, :-1], "dq must be"),
+    (1, lambda t: t.transpose(1, 2), "dk must be"),
+    (2, lambda t: t[:1], "dv must be"),
+    (9, lambda t: t[:, :-1], "rq must be"),
+    (10, lambda t: t.double(), "rk must be"),
+])
+def test_backward_refuses_wrong_gradients_and_rstd(i, change, msg):
+    """The kernels index every operand by the inputs' shape: anything else is refused on the
+    host (the CPU tensors of a well-formed call are refused as such)."""
+    q, k, v, wq, wk, cos, sin = _inputs(dtype=torch.bfloat16)
+    args = [q.transpose(1, 2), k.transpose(1, 2), v.transpose(1, 2), q, k, wq, wk, cos, sin,
+            torch.rand(q.shape[:3]), torch.rand(k.shape[:3])]
+    with pytest.raises(qp.QKPrologueInputError, match="ROCm GPU"):
+        qp.qk_norm_rope_bwd(*args)
+    args[i] = change(args[i])
+    with pytest.raises(qp.QKPrologueInputError, match=msg):
+        qp.qk_norm_rope_bwd(*args)

@@ -103,10 +103,18 @@ def _fwd(q_raw, k_raw, v_raw, wq, wk, cos, sin, eps):
 def _bwd(dq, dk, dv, q_raw, k_raw, wq, wk, cos, sin, rq, rk):
     B, T, Hq, D = q_raw.shape
     Hkv = k_raw.shape[2]
+    for name, t, H in (("dq", dq, Hq), ("dk", dk, Hkv), ("dv", dv, Hkv)):
+        if t.shape != (B, H, T, D) or t.device != q_raw.device:
+            raise QKPrologueInputError(f"{name} must be [B, H, T, D] on the inputs' device")
+    for name, t, H in (("rq", rq, Hq), ("rk", rk, Hkv)):
+        if t.shape != (B, T, H) or t.dtype != torch.float32 or t.device != q_raw.device:
+            raise QKPrologueInputError(f"{name} must be the forward's fp32 [B, T, H] rstd")
+    _check(q_raw, k_raw, k_raw, wq, wk, cos, sin)
     dev = q_raw.device
     ct, st, tab = _tables(cos, sin, T, dev)
     wq32, wk32 = wq.float().contiguous(), wk.float().contiguous()
     dq, dk, dv = (t.to(torch.bfloat16).contiguous() for t in (dq, dk, dv))
+    rq, rk = rq.contiguous(), rk.contiguous()
     dq_raw = torch.empty_like(q_raw)
     dk_raw = torch.empty_like(k_raw)
     dv_raw = torch.empty_like(k_raw)
