@@ -158,6 +158,29 @@ def test_saved_tensors_hooks_and_version_checks():
         o.float().sum().backward()
 
 
+@pytest.mark.parametrize("path", PATHS)
+def test_saved_tensors_handed_back_strided(path):
+    """Saved-tensor hooks may hand the forward's results back with other strides: the
+    gradients are those of the values, as the ops give them."""
+    announce(f"native path strided saved tensors {path}")
+    ins, native, _ = PATHS[path]()
+    want = _grads(native, ins)
+    n = []
+
+    def pack(t):
+        n.append(t)
+        return len(n) - 1, t
+
+    def unpack(it):
+        i, t = it
+        of_forward = i >= 6 if path == "prologue" else i in (3, 4)   # rq, rk / o, M
+        return t.transpose(0, 1).contiguous().transpose(0, 1) if of_forward else t
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        got = _grads(native, ins)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 def test_calls_on_a_side_stream_and_in_threads():
     """Each call runs on its caller's current stream; concurrent threads do not disturb one
     another's results."""

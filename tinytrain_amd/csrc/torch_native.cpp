@@ -104,10 +104,8 @@ bool all_int(at::IntArrayRef sizes) {
   return true;
 }
 
-// A gradient that the native backward may read as it is: plain, and recorded by nothing.
-bool plain_backward(const Tensor &g) {
-  return !c10::GradMode::is_enabled() && plain_mode() && plain_tensor(g);
-}
+// A backward pass that nothing records or traces.
+bool plain_backward() { return !c10::GradMode::is_enabled() && plain_mode(); }
 
 template <class Sig>
 const c10::TypedOperatorHandle<Sig> op(const char *name) {
@@ -159,10 +157,15 @@ Grads3 attn_bwd(const Tensor &q, const Tensor &k, const Tensor &v, const Tensor 
   return {dq, dk, dv};
 }
 
-// What the native backward takes for the gradient of output o: o's shape, type and device
-// (the custom op raises for anything else).
-bool matches(const Tensor &g, const Tensor &o) {
-  return g.sizes() == o.sizes() && g.scalar_type() == o.scalar_type() && g.device() == o.device();
+// A gradient of shape `sizes` and type dt beside q; any strides (it is made contiguous).
+bool grad_of(const Tensor &g, const Tensor &q, at::IntArrayRef sizes, at::ScalarType dt) {
+  return plain_tensor(g) && g.sizes() == sizes && g.scalar_type() == dt && g.device() == q.device();
+}
+
+// A saved tensor as the forward made it: saved-tensor hooks may hand back others, which the
+// custom op makes contiguous or refuses.
+bool saved_as(const Tensor &t, const Tensor &q, at::IntArrayRef sizes, at::ScalarType dt) {
+  return grad_of(t, q, sizes, dt) && t.is_contiguous();
 }
 
 struct FlashAttn : torch::autograd::Function<FlashAttn> {
@@ -177,8 +180,12 @@ struct FlashAttn : torch::autograd::Function<FlashAttn> {
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
     const Tensor &g = grads[0];
-    Grads3 d = plain_backward(g) && matches(g, s[3]) && takes_attn(s[0], s[1], s[2]) &&
-                       plain_tensor(s[3]) && plain_tensor(s[4])
+    const Tensor &q = s[0];
+    const bool native = plain_backward() && takes_attn(q, s[1], s[2]) &&
+                        grad_of(g, q, q.sizes(), q.scalar_type()) &&
+                        saved_as(s[3], q, q.sizes(), q.scalar_type()) &&
+                        saved_as(s[4], q, q.sizes().slice(0, 3), at::kFloat);
+    Grads3 d = native
                    ? attn_bwd(s[0], s[1], s[2], s[3], g, s[4])
                    : op<Grads3(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
                                const Tensor &, const Tensor &)>("tinytrain::flash_attn_bwd")
@@ -248,10 +255,13 @@ struct FlashAttnVarlen : torch::autograd::Function<FlashAttnVarlen> {
   static variable_list backward(AutogradContext *ctx, variable_list grads) {
     const auto s = ctx->get_saved_variables();
     const int64_t longest = ctx->saved_data["max_seqlen"].toInt();
-    const Tensor &g = grads[0];
+    const Tensor &g = grads[0], &q = s[0];
+    const bool native = plain_backward() && takes_varlen(q, s[1], s[2], s[5], longest) &&
+                        grad_of(g, q, q.sizes(), q.scalar_type()) &&
+                        saved_as(s[3], q, q.sizes(), q.scalar_type()) &&
+                        saved_as(s[4], q, q.sizes().slice(0, 2), at::kFloat);
     Grads3 d =
-        plain_backward(g) && matches(g, s[3]) && takes_varlen(s[0], s[1], s[2], s[5], longest) &&
-                plain_tensor(s[3]) && plain_tensor(s[4])
+        native
             ? varlen_bwd(s[0], s[1], s[2], s[3], g, s[4], s[5], longest)
             : op<Grads3(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
                         const Tensor &, const Tensor &, const Tensor &, c10::SymInt)>(
@@ -386,10 +396,15 @@ struct QkNormRope : torch::autograd::Function<QkNormRope> {
     const auto s = ctx->get_saved_variables();
     const Prologue p{s[0], s[1], s[1], s[2], s[3], s[4], s[5]};
     const Tensor &gq = grads[0], &gk = grads[1], &gv = grads[2];
-    const bool native = plain_backward(gq) && plain_tensor(gk) && plain_tensor(gv) && p.takes() &&
-                        plain_tensor(s[6]) && plain_tensor(s[7]) &&
-                        gq.scalar_type() == at::kBFloat16 && gk.scalar_type() == at::kBFloat16 &&
-                        gv.scalar_type() == at::kBFloat16;
+    const Tensor &q = s[0], &k = s[1];
+    bool native = plain_backward() && p.takes();
+    if (native) {
+      const int64_t B = q.size(0), T = q.size(1), Hq = q.size(2), D = q.size(3), Hkv = k.size(2);
+      const auto bf = at::kBFloat16;
+      native = grad_of(gq, q, {B, Hq, T, D}, bf) && grad_of(gk, q, {B, Hkv, T, D}, bf) &&
+               grad_of(gv, q, {B, Hkv, T, D}, bf) && saved_as(s[6], q, {B, T, Hq}, at::kFloat) &&
+               saved_as(s[7], q, {B, T, Hkv}, at::kFloat);
+    }
     Grads5 d = native ? prologue_bwd(gq, gk, gv, p, s[6], s[7])
                       : op<Grads5(const Tensor &, const Tensor &, const Tensor &, const Tensor &,
                                   const Tensor &, const Tensor &, const Tensor &, const Tensor &,
