@@ -10,6 +10,8 @@ op names, schemas, fake shapes, autograd registration and loud failure modes
 import ctypes
 import math
 import re
+import subprocess
+import warnings
 from pathlib import Path
 
 import pytest
@@ -307,6 +309,47 @@ def test_missing_library_raises(monkeypatch, tmp_path):
     monkeypatch.setattr(_lib, "LIB_PATH", tmp_path / "libttfa.so")
     with pytest.raises(_lib.LibraryNotBuilt, match="missing"):
         _lib.load()
+
+
+@needs_lib
+@pytest.mark.parametrize("content", [None, b"not a library"])
+def test_ops_serve_without_the_native_extension(content, tmp_path, monkeypatch):
+    """The extension is built against one torch: where it is missing or does not load, calls
+    are handed on to the custom ops, with one warning."""
+    path = tmp_path / "_ttfa_torch.so"
+    if content is not None:
+        path.write_bytes(content)
+    monkeypatch.setattr(_lib, "_native", None)
+    monkeypatch.setattr(_lib, "NATIVE_PATH", path)
+    with pytest.warns(RuntimeWarning, match="does not load"):
+        native = _lib.native()
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert _lib.native() is native
+    assert native.flash_attn(1, 2, 3) is None and native.qk_norm_rope(*range(8)) is None
+    assert native.flash_attn_varlen(*range(5)) is None and native.flash_attn_decode(*range(4)) is None
+
+
+def test_library_is_linked_where_the_extension_does_not_build(tmp_path, monkeypatch):
+    from tinytrain_amd import build
+
+    def run(cmd, **_):
+        Path(cmd[cmd.index("-o") + 1]).write_bytes(b"")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+
+    def no_headers():
+        raise RuntimeError("g++ failed for torch_native.cpp")
+
+    monkeypatch.setattr(build, "LIB", tmp_path / "libttfa.so")
+    monkeypatch.setattr(build, "NATIVE", tmp_path / "_ttfa_torch.so")
+    monkeypatch.setattr(build, "OBJ_DIR", tmp_path / "obj")
+    monkeypatch.setattr(build, "_generate", lambda: None)
+    monkeypatch.setattr(build, "_compile_native", no_headers)
+    monkeypatch.setattr(build.subprocess, "run", run)
+    build.NATIVE.write_bytes(b"of another build")
+    with pytest.raises(RuntimeError, match="torch_native"):
+        build.build()
+    assert build.LIB.exists() and not build.NATIVE.exists()
 
 
 # ------------------------------------------------------------------ varlen entry points

@@ -120,14 +120,19 @@ def build(verbose: bool = False, extra_flags: list[str] | None = None) -> Path:
     with ThreadPoolExecutor(max_workers=min(8, len(srcs))) as ex:
         native = ex.submit(_compile_native)
         objs = list(ex.map(lambda s: _compile(s, extra), srcs))
-        native_obj = native.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [_hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objs), "-o", str(tmp)]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB)
-    _link_native(native_obj)
+    # libttfa.so stands by itself (the C ABI needs no torch): it is there even where the
+    # extension does not build, and no extension of another libttfa.so is left beside it.
+    try:
+        _link_native(native.result())
+    except BaseException:
+        NATIVE.unlink(missing_ok=True)
+        raise
     if verbose:
         print(f"built {LIB} from {len(srcs)} sources, and {NATIVE.name}")
     return LIB
