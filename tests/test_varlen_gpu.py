@@ -116,6 +116,38 @@ def test_varlen_autograd_and_opcheck():
                           test_utils=("test_schema", "test_faketensor"))
 
 
+@pytest.mark.parametrize("lens, D", [
+    ([5, 0, 300, 129, 1], 64),
+    ([40 + (37 * i) % 290 for i in range(65)], 128),
+])
+def test_overstated_max_seqlen(lens, D):
+    """max_seqlen above the longest sequence changes nothing; calls of half the sequences give
+    the same bits too, and skipped sequences (bounds that decrease, or end past the tokens)
+    beside the others leave them as they are."""
+    announce(f"varlen overstated max_seqlen n_seq={len(lens)} D={D}")
+    q, k, v, do, cu = (t.to(DEV) for t in _inputs(lens, 4, 2, D, seed=6))
+    total, long_one = sum(lens), max(lens)
+
+    def run(a, z, longest, bounds=None):
+        part = lambda t: t[:, a:z].contiguous()  # noqa: E731
+        ins = [part(t) for t in (q, k, v)]
+        c = cu[(cu >= a) & (cu <= z)] - a if bounds is None else bounds
+        o, M = flash_attn_varlen_fwd(*ins, c.contiguous(), longest)
+        return (o, M, *flash_attn_varlen_bwd(*ins, o, part(do), M, c.contiguous(), longest))
+
+    want = run(0, total, long_one)
+    for more in (long_one + 1, 4 * long_one + 131):
+        for a, b in zip(run(0, total, more), want):
+            assert torch.equal(a, b)
+    at = int(cu[len(lens) // 2])
+    for a, z in ((0, at), (at, total)):
+        for x, w in zip(run(a, z, long_one), want):
+            assert torch.equal(x, w[:, a:z])
+    skipped = torch.cat([cu, cu.new_tensor([total - 1, total + 9])])
+    for x, w in zip(run(0, total, long_one, skipped), want):
+        assert torch.equal(x, w)
+
+
 @pytest.mark.parametrize("D", [64, 128])
 def test_sequence_longer_than_max_seqlen(D):
     """A sequence longer than max_seqlen is processed as its first max_seqlen tokens by

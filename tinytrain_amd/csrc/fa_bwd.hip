@@ -295,9 +295,9 @@ __global__ __launch_bounds__(256, (D == 64 ? 3 : 2)) void fa_bwd_dq_bf16_kernel(
 }
 
 // Packed variable-length sequences ([H, total, D], sequence s at rows cu_seqlens[s] ..
-// cu_seqlens[s+1]-1 of every head; LSE / Delta [H, total]).  Workgroup -> (rank, sequence,
-// query head), rank r being row tile max_tiles - 1 - r, longest first over all sequences (the
-// forward's order); invalid sequence bounds are skipped.
+// cu_seqlens[s+1]-1 of every head; LSE / Delta [H, total]).  Workgroup -> (tile rank,
+// sequence, query head), rank-major, longest row tiles first; invalid sequence bounds
+// are skipped.
 template <int D>
 __global__ __launch_bounds__(256, (D == 64 ? 3 : 2)) void fa_bwd_dq_varlen_bf16_kernel(
     const bf16 *__restrict__ Q, const bf16 *__restrict__ K, const bf16 *__restrict__ V,
@@ -313,8 +313,8 @@ __global__ __launch_bounds__(256, (D == 64 ? 3 : 2)) void fa_bwd_dq_varlen_bf16_
   if (c0 < 0 || c1 < c0 || c1 > total) return;
   const int T = min(c1 - c0, max_seqlen);  // the forward's clamp
   const int n_tiles = (T + P::BM - 1) / P::BM;
-  const int qt = (max_seqlen + P::BM - 1) / P::BM - 1 - rank;
-  if (qt >= n_tiles) return;
+  if (rank >= n_tiles) return;
+  const int qt = n_tiles - 1 - rank;
   const int hk = h / (Hq / Hkv);
   const int64_t qb = ((int64_t)h * total + c0) * D, kb = ((int64_t)hk * total + c0) * D;
   const int64_t rb = (int64_t)h * total + c0;

@@ -238,9 +238,9 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dkdv_split_bf16_kernel<64>(
 }
 
 // Packed variable-length sequences ([H, total, D] per tensor, sequence s at rows
-// cu_seqlens[s] .. cu_seqlens[s+1]-1 of every head): the same stage body per (rank,
-// sequence, KV head), rank-major: rank r is the key tile with max_tiles - r query tiles to
-// visit, so workgroups come longest first over all sequences; one without such a tile exits at
+// cu_seqlens[s] .. cu_seqlens[s+1]-1 of every head): the same stage body per (key tile,
+// sequence, KV head), key-tile-major so every sequence's longest key tiles (tile 0 sees
+// all of its query rows) are dispatched first; a key tile past a sequence's end exits at
 // once.  Sequences whose bounds are not 0 <= cu[s] <= cu[s+1] <= total are skipped, and a
 // sequence longer than max_seqlen is processed as its first max_seqlen tokens (the
 // forward's clamp).  The per-sequence head view restricts every load to the sequence's
@@ -254,13 +254,12 @@ __global__ __launch_bounds__(256, 2) void fa_bwd_dkdv_varlen_bf16_kernel<64>(
     float scale_log2, float scale) {
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
   const int per_rank = n_seq * Hkv;
-  const int rank = blockIdx.x / per_rank, rem = blockIdx.x - rank * per_rank;
+  const int kt = blockIdx.x / per_rank, rem = blockIdx.x - kt * per_rank;
   const int s = rem / Hkv, hk = rem - s * Hkv;
   const int c0 = cu_seqlens[s], c1 = cu_seqlens[s + 1];
   if (c0 < 0 || c1 < c0 || c1 > total) return;
   const int T = min(c1 - c0, max_seqlen);
-  const int kt = (T + 127) / 128 - ((max_seqlen + 127) / 128 - rank);
-  if (kt < 0) return;
+  if (kt >= (T + 127) / 128) return;
   const int G = Hq / Hkv;
   const int64_t hs = (int64_t)total * 64, kvb = (int64_t)hk * hs + (int64_t)c0 * 64;
   const int64_t q0 = (int64_t)hk * G;
