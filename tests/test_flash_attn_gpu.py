@@ -333,6 +333,30 @@ def test_split_forward(B, H, H_kv, T, D, split):
     assert ((o.float() - po.float()).norm() <= 2 ** -8 * po.float().norm()).item()
 
 
+@pytest.mark.parametrize("B, H, T", [
+    (1, 2, 64), (1, 2, 65),          # rows of four key blocks, of five
+    (9, 4, 100), (1, 37, 100),       # 252 and 259 row blocks
+    (1, 23, 200), (4, 6, 193),       # 299 and 312
+    (2, 13, 300), (3, 9, 300),       # 494 and 513
+    (5, 3, 1030), (2, 8, 1030),      # 975 and 1040
+])
+def test_fp32_forward_waves(B, H, T):
+    """fp32 at D = 128: both sides of every bound between eight and four waves per workgroup,
+    against the fp64 oracle; every element written."""
+    announce(f"fp32 forward waves B={B} H={H} T={T}")
+    D = 128
+    q, k, v, do = make_custom(B, H, H, T, D, torch.float32, seed=T)
+    want = attention_fwd(q, k, v, dtype=torch.float64)
+    q, k, v = (t.to(DEV) for t in (q, k, v))
+    o, M = torch.full_like(q, float("nan")), torch.full((B, H, T), float("nan"), device=DEV)
+    _lib.check(_lib.load().ttfa_fwd(*[t.data_ptr() for t in (q, k, v, o, M)], B, H, H, T, D,
+                                    _lib.TTFA_F32, 1.0 / math.sqrt(D),
+                                    torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert_close_abs("O", o, want[0], TOL[torch.float32])
+    assert_close_abs("LSE", M, want[1], TOL_LSE)
+
+
 @pytest.mark.parametrize("B, H, H_kv, T, D, split", [
     (1, 8, 1, 96, 128, True),      # 48 items against 8
     (2, 12, 4, 100, 128, False),   # 21 items: fewer than four rounds of the waves to save

@@ -8,7 +8,7 @@
 // operands, fp32 accumulate) and the exponentials are the accurate expf / logf.
 //
 // Work split: 16-row blocks.  A workgroup owns one 16-row query block (forward, dQ) or
-// one 16-key block (dK/dV); its waves (eight at D = 64, four at D = 128) take the
+// one 16-key block (dK/dV); its waves (eight or four, see below) take the
 // block's partner blocks round-robin (the key blocks at or below the diagonal, or the
 // query blocks at or above it over the head group), each with its own partial result,
 // and the partials are merged through LDS in wave order, so results do not depend on
@@ -22,7 +22,7 @@
 // which saturates the per-CU load pipeline long before HBM or L2.)  The LDS writes come
 // first and the next block's loads go into the same registers: loads issued before the
 // writes need a second set and a move per register, which cost the forward 21.4 -> 23.3 us
-// at 2x8/2x500 and 105.8 -> 114.7 at 2x16/8x900 (D = 128).
+// at 2x8/2x500 and 105.8 -> 114.7 at 2x16/8x900 (D = 128, eight waves).
 //
 // MFMA 16x16x4 lane layout (lane = 16 j + n): A supplies A[n][j], B supplies B[j][n],
 // and register r of the result is D[4 j + r][n].  A contraction over D features uses
@@ -41,14 +41,11 @@ namespace {
 
 constexpr int kF32Rows = 16;  // rows per block
 
-// Waves per workgroup.  Forward: eight (two per SIMD, so one wave's dependent product chain
-// overlaps the other's; 193 registers at D = 128, where four waves and two workgroups per CU
-// took 25.8 us at 2x8/2x500 and 131 at 2x16/8x900 against 23.7 and 115: a workgroup's
-// serial chain halves and the second round balances the first).  Backward: eight at
-// D = 64, four at D = 128, whose 340 operand registers do not leave room for two waves per
-// SIMD (with K and V re-read from LDS tiles eight fit, spilling 24: 67.2 us against 68.2 at
-// 2x8/2x500, but 27.5 against 21.4 at 4x6/2x130).
-constexpr int kF32FwdWaves = 8;
+// Waves per workgroup.  Forward: eight at D = 64, eight or four at D = 128
+// (f32_fwd_eight_waves).  Backward: eight at D = 64, four at D = 128, whose 340 operand
+// registers do not leave room for two waves per SIMD (with K and V re-read from LDS tiles
+// eight fit, spilling 24: 67.2 us against 68.2 at 2x8/2x500, but 27.5 against 21.4 at
+// 4x6/2x130).
 template <int D>
 constexpr int f32_waves() {
   return D == 64 ? 8 : 4;
@@ -189,15 +186,15 @@ __device__ __forceinline__ float *wave_tiles(float *lds, int wave) {
 
 }  // namespace
 
-template <int D>
-__global__ __launch_bounds__(64 * kF32FwdWaves) void fa_fwd_f32_kernel(const float *__restrict__ Q,
-                                                         const float *__restrict__ K,
-                                                         const float *__restrict__ V,
-                                                         float *__restrict__ O,
-                                                         float *__restrict__ LSE, int Hq,
-                                                         int Hkv, int T, int n_bh,
-                                                         float scale) {
-  constexpr int NW = kF32FwdWaves, TPW = 2;
+template <int D, int NW>
+__global__ __launch_bounds__(64 * NW) void fa_fwd_f32_kernel(const float *__restrict__ Q,
+                                                             const float *__restrict__ K,
+                                                             const float *__restrict__ V,
+                                                             float *__restrict__ O,
+                                                             float *__restrict__ LSE, int Hq,
+                                                             int Hkv, int T, int n_bh,
+                                                             float scale) {
+  constexpr int TPW = 2;
   __shared__ __attribute__((aligned(16))) float lds[NW * TPW * tile_floats<D>()];
   __shared__ float pm[NW][kF32Rows], pl[NW][kF32Rows];
   const int n_blk = (T + kF32Rows - 1) / kF32Rows;
@@ -628,18 +625,32 @@ static F32Bwd bwd_args(const void *q, const void *k, const void *v, const void *
                 Hq, Hkv, T, scale};
 }
 
+// D = 128 forward: eight waves per workgroup, one workgroup per CU (135 KB of LDS), or four and
+// two.  Eight halve a row block's serial chain of key blocks, so they win while the launch is
+// about one round of the 256 CUs, or long rows make the chain what counts; beyond that they
+// halve the row blocks in flight, and rows of up to four key blocks leave half of them idle.
+// Measured, us, eight against four waves (n row blocks, T):
+//   T 100: n 252 7.3 / 7.6, 280 9.8 / 8.1      T 64: n 256 6.0 / 5.6, 512 10.4 / 7.5
+//   T 200: n 260 10.0 / 11.2, 312 11.4 / 11.2, 468 14.2 / 12.6
+//   T 280: n 504 16.2 / 16.8, 576 20.2 / 16.9  T 500: n 512 20.9 / 24.0, 576 26.4 / 24.6
+//   T 1000: n 504 32.9 / 42.7, 1134 72.4 / 68.4
+//   T 2000: n 500 56.9 / 78.5, 1000 107.9 / 114.3, 1500 159 / 155
+// and up to twice as far apart as n grows (T 64, n 3000: 64.3 / 37.2; T 128, n 4096: 45.7 / 30.7).
+static bool f32_fwd_eight_waves(int64_t n, int T) {
+  return T > 64 && n <= (T <= 128 ? 256 : T <= 256 ? 304 : T <= 1024 ? 512 : 1024);
+}
+
 hipError_t launch_fwd_f32(const void *q, const void *k, const void *v, void *o, float *lse,
                           int B, int Hq, int Hkv, int T, int D, float scale, hipStream_t stream) {
-  const dim3 grid(blocks_grid(B * Hq, T)), block = dim3(64 * kF32FwdWaves);
-  if (D == 64)
-    fa_fwd_f32_kernel<64><<<grid, block, 0, stream>>>((const float *)q, (const float *)k,
-                                                      (const float *)v, (float *)o, lse, Hq,
-                                                      Hkv, T, B * Hq, scale);
-  else
-    fa_fwd_f32_kernel<128><<<grid, block, 0, stream>>>((const float *)q, (const float *)k,
-                                                       (const float *)v, (float *)o, lse, Hq,
-                                                       Hkv, T, B * Hq, scale);
-  return hipGetLastError();
+  auto go = [&](auto kern, int waves) {
+    kern<<<dim3(blocks_grid(B * Hq, T)), dim3(64 * waves), 0, stream>>>(
+        (const float *)q, (const float *)k, (const float *)v, (float *)o, lse, Hq, Hkv, T, B * Hq,
+        scale);
+    return hipGetLastError();
+  };
+  if (D == 64) return go(fa_fwd_f32_kernel<64, 8>, 8);
+  return f32_fwd_eight_waves(blocks_grid(B * Hq, T), T) ? go(fa_fwd_f32_kernel<128, 8>, 8)
+                                                        : go(fa_fwd_f32_kernel<128, 4>, 4);
 }
 
 hipError_t launch_bwd_dq_f32(const void *q, const void *k, const void *v, const void *o,
