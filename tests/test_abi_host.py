@@ -163,11 +163,15 @@ def test_bwd_workspace_bytes():
     lib = _lib.load()
     for B, Hq, Hkv, T, D in [(16, 12, 12, 1024, 64), (32, 12, 4, 1024, 64), (4, 16, 8, 4096, 128),
                              (1, 16, 8, 16384, 128), (32, 8, 2, 512, 128), (1, 8, 2, 512, 128),
-                             (1, 8, 2, 4500, 64), (3, 2, 2, 1, 64)]:
+                             (1, 8, 2, 4500, 64), (3, 2, 2, 1, 64),
+                             # D = 64: a piece saves less than its partials cost
+                             (24, 12, 4, 129, 64), (8, 4, 4, 800, 64), (2, 12, 12, 723, 64),
+                             (5, 4, 4, 723, 64), (48, 8, 2, 129, 64), (16, 12, 4, 400, 64)]:
         n = lib.ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, _lib.TTFA_BF16)
         assert n == 4 * -(-B * Hq * T // 4) * 4, (B, Hq, Hkv, T, D)
     for B, Hq, Hkv, T, D in [(2, 8, 2, 512, 128), (3, 8, 2, 333, 128), (1, 8, 2, 8000, 128),
-                             (4, 8, 2, 1000, 64), (2, 8, 1, 3000, 64)]:
+                             (4, 8, 2, 1000, 64), (2, 8, 1, 3000, 64), (16, 8, 2, 129, 64),
+                             (12, 12, 4, 400, 64), (2, 4, 4, 1300, 64)]:
         n = lib.ttfa_bwd_workspace_bytes(B, Hq, Hkv, T, D, _lib.TTFA_BF16)
         part = n - 4 * -(-B * Hq * T // 4) * 4
         slots = 512 if D == 64 else 256

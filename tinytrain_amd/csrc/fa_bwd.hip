@@ -444,10 +444,14 @@ static hipError_t launch_dkdv(const void *q, const void *k, const void *v, const
 //             16x8/2x512 78 -> 61, 2x16/8x1500 122 -> 107, 1x8/2x8000 939 -> 513
 //   D = 64:   4x8/2x1000 82.5 -> 47, 2x12/4x2000 127 -> 76, 8x12/4x512 41 -> 36
 // Around the chosen size the time is flat (4x8/2x1000 with 2 .. 8 stages: 64.6-67.2).  It has
-// to save more stages than the partials cost: about 4 at D = 128; at D = 64, where two
-// workgroups share a CU and an idle device already runs each of them faster, more than half
-// of the list (3x12/12x900, 8 -> 4 stages, was 40.3 -> 43.6, and 2x12/12x2000, 16 -> 8,
-// 77.1 -> 79.3).
+// to save more stages than the partials cost: 4 at D = 128 (the least gain of 224 such shapes:
+// 4x16/8x300, 6 -> 2 stages, 36.3 -> 35.1).  At D = 64, where two workgroups share a CU and an
+// idle device already runs each of them faster, more than half of the list, and against every
+// 64 KB partial a stage is cheap: over 195 shapes with such a list the gain was about
+// 1.44 (longest list - longest piece) - 0.02 partials - 2.7 us.  So 80 stages saved have to
+// outweigh 240 partials more than there are: 24x12/4x129 (6 -> 2 stages, 480 partials) would be
+// 25.1 -> 31.7 us, 8x4/4x800 (7 -> 2, 512) 34.0 -> 39.9, 2x12/12x900 (8 -> 2, 480) 37.0 -> 41.5;
+// 12x12/4x400 (12 -> 3, 480) is 40.5 -> 38.4, 16x8/2x129 (8 -> 2, 192) 25.5 -> 23.0.
 // A single sequence keeps the unsplit sums, the bits of the packed entry point, except at
 // D = 128 above T = 1792, where those differ by the 256-row kernels too.
 DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
@@ -459,12 +463,15 @@ DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
   if (units > slots || longest > (1 << 24)) return none;
   auto pays = [&](int64_t st) { return longest >= (D == 64 ? 2 * st + 2 : st + 4); };
   int split_tiles = 0;
+  int64_t longest_piece = 0;
   auto pieces = [&](int64_t st) {
     int64_t p = 0;
     DkvTiles t(n, G, (int)st);
-    for (split_tiles = 0; t.kt < n; t.next()) {
+    for (split_tiles = 0, longest_piece = 0; t.kt < n; t.next()) {
       p += t.n;
       split_tiles += t.n > 1;
+      const int64_t stages = ((int64_t)G * (n - t.kt) + t.n - 1) / t.n;
+      longest_piece = stages > longest_piece ? stages : longest_piece;
     }
     return p;
   };
@@ -473,6 +480,7 @@ DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
   for (st = st < 2 ? 2 : st; pays(st); st += 1 + st / 32)
     if ((p = pieces(st)) * units <= slots) break;
   if (!pays(st)) return none;
+  if (D == 64 && 80 * (longest - longest_piece) < p * units + 240) return none;
   return {(int)st, (int)p, split_tiles};
 }
 
