@@ -182,6 +182,25 @@ def test_bwd_workspace_bytes():
 
 
 @needs_lib
+def test_decode_workspace_bytes():
+    """Partials of every chunk of every row.  A call of up to 512 KV heads in all with long
+    caches has at least about 400 workgroups, so that a long cache among short ones is read by
+    more than one; the size follows the exact shape, not its order."""
+    chunks = lambda B, Hkv, L, D: (_lib.load().ttfa_decode_workspace_bytes(B, Hkv, Hkv, 1, L, D)  # noqa: E731
+                                   // (B * Hkv * (D + 2) * 4))
+    for B, Hkv, L, D in [(32, 8, 16384, 128), (32, 8, 4096, 128), (16, 8, 4096, 128), (16, 2, 4096, 128),
+                         (2, 1, 300000, 128), (64, 4, 16384, 64), (24, 12, 4096, 64), (9, 12, 2048, 64)]:
+        n = chunks(B, Hkv, L, D)
+        assert 409 <= n * B * Hkv <= 640, (B, Hkv, L, D, n)
+    for B, Hkv, L, D in [(64, 8, 16384, 128), (52, 8, 4096, 64), (33, 8, 2016, 128), (1, 2, 512, 64)]:
+        assert chunks(B, Hkv, L, D) == 1
+    assert chunks(1, 8, 16384, 128) == 32
+    assert chunks(1, 1, 100000, 64) == 512                        # at most
+    small, large = (_lib.load().ttfa_decode_workspace_bytes(B, 2, 2, 1, 4818, 128) for B in (25, 26))
+    assert small > large                                          # 10 chunks against 9
+
+
+@needs_lib
 def test_check_raises_with_message():
     with pytest.raises(_lib.TTFAError, match="head dim"):
         _lib.check(_fwd(D=80))

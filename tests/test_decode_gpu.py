@@ -7,6 +7,8 @@
 * decoding the last rows of a sequence agrees with the batched forward kernel on the
   whole sequence;
 * run-to-run bitwise determinism and the torch.library op checks;
+* every bound of the rule that splits a call, and rows that do not depend on other caches;
+* NaN keys, which reach exactly the rows that see them;
 * a workspace reused across shapes with leftovers in it, and HIP-graph replays with new
   inputs, both bitwise equal to fresh eager calls.
 """
@@ -56,21 +58,41 @@ def test_decode_matches_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
     assert_close_abs("LSE", lse.cpu()[fin], want_lse[fin], TOL_LSE)
 
 
-@pytest.mark.parametrize("B, Hq, Hkv, Tq, Lmax, D, lens", [
-    (3, 4, 2, 1, 512, 128, [512, 33, 0]),       # 16 blocks: one workgroup per head, one launch
-    (2, 4, 2, 3, 513, 128, [513, 2]),           # 17 blocks: split, two waves per workgroup
-    (2, 2, 1, 1, 512, 64, [511, 480]),
-    (1, 2, 1, 2, 545, 64, [545]),               # D = 64 split: four waves per workgroup
-    (4, 16, 16, 1, 2017, 128, [2017, 2016, 1, 600]),   # 64 * 64 blocks: the last two-wave shape
-    (4, 16, 16, 1, 2049, 128, [2049, 31, 2048, 97]),   # 64 * 65 blocks: four waves
-    (40, 8, 8, 4, 700, 128, [700 - 17 * i for i in range(40)]),  # 320 heads: one chunk each
-    (2, 32, 1, 1, 1000, 128, [1000, 65]),       # 32 query columns fill the merge stage
-    (1, 8, 2, 8, 16500, 64, [16391]),           # many chunks of two blocks per head
+def _uneven(B, L, step):
+    return [max(L - step * i, 0) for i in range(B)]
+
+
+@pytest.mark.parametrize("B, Hq, Hkv, Tq, Lmax, D, lens, chunks", [
+    (3, 4, 2, 1, 512, 128, [512, 33, 0], 1),            # 16 blocks: one launch
+    (2, 2, 1, 1, 512, 64, [511, 480], 1),
+    (2, 4, 2, 3, 513, 128, [513, 2], 9),                # 17: a block for every wave of a chunk
+    (1, 2, 1, 2, 545, 64, [545], 5),
+    (2, 32, 1, 1, 1000, 128, [1000, 65], 16),           # 32 query columns fill the merge stage
+    (1, 16, 8, 1, 5000, 128, [4999], 32),               # one sequence: 256 workgroups
+    (2, 16, 8, 1, 5000, 128, [4999, 31], 32),           # two: 512
+    (1, 8, 2, 8, 16500, 64, [16391], 129),              # many chunks of few blocks per head
+    (16, 4, 2, 1, 1000, 128, _uneven(16, 1000, 61), 16),    # 32 heads: chunks of two blocks
+    (17, 4, 2, 1, 1000, 128, _uneven(17, 1000, 61), 15),    # 34: of a share each, 3 blocks
+    (17, 4, 2, 2, 11500, 128, _uneven(17, 11500, 767), 15),  # a share of 24: four waves
+    (17, 4, 2, 1, 11000, 128, _uneven(17, 11000, 733), 15),  # of 23: two
+    (26, 4, 2, 1, 1200, 128, _uneven(26, 1200, 47), 9),  # 468 of 512 slots
+    (32, 24, 3, 1, 700, 64, _uneven(32, 700, 22), 5),    # 480
+    (54, 8, 2, 1, 700, 64, _uneven(54, 700, 13), 4),     # 432
+    (65, 6, 3, 1, 800, 128, _uneven(65, 800, 12), 3),    # 390 would leave a fifth empty: 585
+    (102, 4, 4, 1, 2048, 64, _uneven(102, 2048, 20), 2),  # 408 heads of 64 blocks: two chunks
+    (102, 4, 4, 1, 2016, 64, _uneven(102, 2016, 20), 1),  # of 63: one, eight waves
+    (103, 4, 4, 1, 2048, 64, _uneven(103, 2048, 20), 1),  # 412 heads
+    (103, 4, 4, 1, 1504, 64, _uneven(103, 1504, 15), 1),  # 47 blocks: four waves
+    (40, 8, 8, 4, 700, 128, _uneven(40, 700, 17), 1),
 ])
-def test_decode_splits_match_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
+def test_decode_splits_match_oracle(B, Hq, Hkv, Tq, Lmax, D, lens, chunks):
     """Both sides of every rule that picks a call's workgroups per head and waves per
-    workgroup, with uneven and empty caches."""
+    workgroup, with uneven and empty caches, every second head group's last column among them."""
+    from tinytrain_amd import _lib
+
     announce(f"decode splits B={B} Hq={Hq} Hkv={Hkv} Tq={Tq} Lmax={Lmax} D={D} lens={lens[:4]}")
+    nbytes = _lib.load().ttfa_decode_workspace_bytes(B, Hq, Hkv, Tq, Lmax, D)
+    assert nbytes == B * Hq * Tq * chunks * (D + 2) * 4
     q, k, v = _inputs(B, Hq, Hkv, Tq, Lmax, D)
     lens_t = torch.tensor(lens, dtype=torch.int32)
     want_o, want_lse = decode_reference(q, k, v, lens)
@@ -80,6 +102,24 @@ def test_decode_splits_match_oracle(B, Hq, Hkv, Tq, Lmax, D, lens):
     seen = torch.isfinite(want_lse)
     assert torch.equal(torch.isfinite(lse.cpu()), seen)
     assert_close_abs("lse", lse.cpu()[seen], want_lse[seen], TOL_LSE)
+
+
+@pytest.mark.parametrize("B, Hkv, L, D", [(17, 2, 2500, 128), (40, 2, 4000, 64), (8, 8, 8000, 128)])
+def test_decode_rows_do_not_depend_on_the_other_caches(B, Hkv, L, D):
+    """A sequence's bits are a function of the call's shape and of its own cache: the same
+    beside full, short or empty caches, whose unused workgroups leave no trace."""
+    announce(f"decode neighbours B={B} Hkv={Hkv} L={L} D={D}")
+    q, k, v = (t.to(DEV) for t in _inputs(B, 2 * Hkv, Hkv, 1, L, D, seed=9))
+    own = [L, L - 1, 33 * 32, 32, 1]
+
+    def run(rest):
+        lens = torch.tensor(own + [rest] * (B - len(own)), dtype=torch.int32, device=DEV)
+        return [t[:len(own)] for t in flash_attn_decode(q, k, v, lens)]
+
+    want = run(L)
+    for rest in (L // 3, 40, 0):
+        for a, b in zip(run(rest), want):
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("Hkv, L, D, lens, at", [

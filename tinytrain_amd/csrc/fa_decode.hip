@@ -8,33 +8,45 @@
 // 0 .. L_b - Tq + i of the cache, O = softmax(q k^T * scale) v, LSE = m + ln(l).
 //
 // Work split (split-K, "flash decoding"): a unit is one (batch, KV head).  Its 32-key blocks
-// in use (its own cache length, not the capacity) are dealt evenly to n_chunks workgroups,
-// and a workgroup's blocks to its waves in turn, so the workgroups of a unit have the same
-// work whatever its length.  Workgroups are numbered chunk-major: consecutive ids, which
-// the hardware deals to the XCDs, are different units, so batches of uneven lengths spread
-// over all XCDs.  All G query heads of the KV head and all Tq rows form the R = G * Tq <= 32
-// query columns of one 32x32 MFMA tile (columns past R repeat valid ones and are not
-// stored), so the K and V bytes are read once for the whole group.
+// in use (its own cache length, not the capacity) are dealt to as many of its n_chunks
+// workgroups as have 2^log2_min of them each, in turn over all of their waves; the others
+// leave an empty partial.  So a long cache among short ones still has every chunk, and a short
+// one few.  The split depends on the call's shape and on the cache's own length alone, never
+// on the other caches, so neighbours do not change a row's bits.
+// Workgroups are numbered chunk-major, each chunk's units turned (chunk_turn): consecutive ids
+// go to the XCDs in turn, and with a multiple of eight units every chunk of a unit would
+// share an XCD (16 caches, every other one 400 of 8000 keys, Hkv 4, D 64: 24.7 -> 17.0 us).
+// All G query heads of the KV head and all Tq rows form the R = G * Tq <= 32 query columns of
+// one 32x32 MFMA tile (columns past R repeat valid ones and are not stored), so the K and V
+// bytes are read once for the whole group.
 //
-// Data path: a wave loads a block's K and V rows straight into its own LDS stage, whole
-// rows in order (16 bytes per lane, 1 KB per instruction), the next block's loads in flight
-// while the current one is computed (the wave waits on its own vmcnt only; no workgroup
-// barriers).  K fragments loaded straight into the MFMA operand registers, 32 bytes from
-// each of 32 rows per instruction, read 8% slower at 32 x 4096 keys.  Per block:
-// S^T = K Q^T, online softmax in the exp2 domain (lazy rescale as in the forward kernel),
-// O^T += V^T P^T.  The waves' partials (unnormalised O, running max m in log2 units, sum l)
-// are merged through LDS, in wave order.  With one chunk the workgroup then writes O and
-// LSE itself; otherwise it writes one fp32 partial per query row, and a second kernel
+// Data path: a wave has one LDS stage, into which a block's K and V rows are loaded directly,
+// whole rows in order (16 bytes per lane, 1 KB per instruction).  The next block's K is
+// requested as soon as this one's is in registers, before the scores, its V after the last V
+// read, so a wave keeps about one block in flight (it waits on its own vmcnt only; no
+// workgroup barriers).  Two stages and the whole next block ahead took twice the LDS, one
+// workgroup per CU at D = 128, for the same time (16 x 4096 keys, 8 heads, four chunks: 54.0
+// us with one stage, 55.1 with two).  K fragments loaded straight into the MFMA operand
+// registers, 32 bytes from each of 32 rows per instruction, read 8% slower at 32 x 4096 keys.
+// Per block: S^T = K Q^T, online softmax in the exp2 domain (lazy rescale as in the forward
+// kernel), O^T += V^T P^T.  The waves' partials (unnormalised O, running max m in log2 units,
+// sum l) are merged through LDS, in wave order.  A unit with one workgroup has its O and LSE
+// written by it; otherwise each writes one fp32 partial per query row, and a second kernel
 // merges the chunks with the log-sum-exp rule.
 //
 // What bounds it: the cache bytes from HBM (a plain read kernel reaches 6.8-7.1 TB/s on
-// MI355X), and for small caches the launches.  Back-to-back time per call, before (one
-// range of keys per wave, four partials per workgroup, always two launches) and now:
-//   B 32, Hkv 8, D 128, lengths 410..4096 of 4096: 73.0 -> 63.9 us (5.0 TB/s)
-//   B 32, Hkv 8, D 128, 4096 keys each:            98.9 -> 90.5 us (5.9 TB/s)
-//   B 1,  Hkv 8, D 128, 16384 keys:                19.5 -> 19.2 us
-//   B 64, Hkv 12, D 64, lengths 200..2000 of 2000: 51.1 -> 44.8 us
-//   B 1,  Hkv 2, D 128, 512 keys:                  11.1 ->  8.3 us (one launch)
+// MI355X), for small caches the launches, and for one long cache among short ones the rate of
+// the CUs that read it (40-60 GB/s each).
+// Back-to-back us per call: with one range of keys per wave, four partials per workgroup and
+// always two launches; with as many chunks as gave 256 workgroups, all used whatever the
+// length (which left a long cache to one or two CUs); now:
+//   B 32, Hkv 8, D 128, 4096 keys each                  99.7   92.5   98.0
+//     lengths 410..4096 of 4096                         69.0   57.4   59.8
+//     one of 4096, the others up to 500                 28.5   36.9   30.5
+//   B 16, Hkv 8, D 128, one of 16384, the others short  45.0   68.1   41.6
+//   B 64, Hkv 12, D 64, lengths 200..2000 of 2000       49.5   44.8   43.0
+//   B 1, Hkv 8, D 128, 16384 keys                       17.0   17.0   16.9
+//   B 1, Hkv 2, D 128, 512 keys                         11.6    9.1    9.1  (one launch)
 #include "fa_bwd.h"  // allow_lds
 #include "fa_common.h"
 #include "fa_kernels.h"
@@ -51,8 +63,7 @@ template <int D>
 struct DecShape {
   static constexpr int KK = D / 16, DB = D / 32, CH = D / 8;
   static constexpr int LOADS = kDecBlock * CH / 64;       // 1 KB DMA blocks per K (V) block
-  static constexpr int VMEM_PER_BLOCK = 2 * LOADS;        // vector memory ops per block
-  static constexpr int WAVE_LDS = 2 * 2 * kDecBlock * D;  // bf16 elements, [stage][K|V]
+  static constexpr int WAVE_LDS = 2 * kDecBlock * D;      // bf16 elements, [K|V]
 };
 
 // s_waitcnt vmcnt(N) (gfx9 encoding: vmcnt bits 3:0 and 15:14; expcnt, lgkmcnt at max)
@@ -63,16 +74,20 @@ __device__ __forceinline__ void wait_vmcnt() {
 }
 
 // One 32-key block of one wave: S^T = K Q^T, mask, online softmax, O^T += V^T P^T.
-template <int D, bool MASK>
+template <int D, bool MASK, class NextK, class WaitV>
 __device__ __forceinline__ void decode_block(const bf16 *Kt, const bf16 *Vt,
                                              const bf16x8 (&qf)[D / 16], f32x16 (&oacc)[D / 32],
                                              float &m_t, float &l_part, float scale_log2, int k0,
-                                             int pos, int L, int lane) {
+                                             int pos, int L, int lane, NextK next_k, WaitV wait_v) {
   using P = DecShape<D>;
   const int lg = lane >> 5;
   bf16x8 kf[P::KK];
 #pragma unroll
   for (int kk = 0; kk < P::KK; ++kk) kf[kk] = lds_read_row8<D, 1>(Kt, lane & 31, 2 * kk + lg);
+  __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the K rows are in registers
+  __builtin_amdgcn_sched_barrier(0);
+  next_k();
+  __builtin_amdgcn_sched_barrier(0);
   f32x16 s = mfma32(kf[0], qf[0], f32x16{});
 #pragma unroll
   for (int kk = 1; kk < P::KK; ++kk) s = mfma32(kf[kk], qf[kk], s);
@@ -109,6 +124,9 @@ __device__ __forceinline__ void decode_block(const bf16 *Kt, const bf16 *Vt,
     pb[m] = pack8(f32x16{p[0], p[1], p[2], p[3], p[4], p[5], p[6], p[7]}, 0);
   }
   l_part += rs;
+  __builtin_amdgcn_sched_barrier(0);
+  wait_v();
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int m = 0; m < 2; ++m) {
     bf16x8 vf[P::DB];
@@ -119,23 +137,47 @@ __device__ __forceinline__ void decode_block(const bf16 *Kt, const bf16 *Vt,
   }
 }
 
+// Workgroups of a unit that have work: its nb blocks, 2^log2_min each at least (a power of two:
+// a quotient would stand between the length's load and the first block's).
+__device__ __forceinline__ int used_chunks(int nb, int n_chunks, int log2_min) {
+  return max(min((nb + (1 << log2_min) - 1) >> log2_min, n_chunks), 1);
+}
+
+// Places by which chunk `chunk` turns its units (n_units >= 8).  Consecutive workgroups go to the
+// XCDs in turn, and those of an XCD to its 32 CUs: 37 = 4 * 8 + 5 moves a unit's chunks to
+// other XCDs and other CUs.  Fewer units have more chunks, whose own numbers do that.
+__device__ __forceinline__ int chunk_turn(int chunk, int n_units) {
+  int turn = chunk * (n_units >= 64 ? 37 : 5);
+  if (n_units < 32) turn &= 7;
+  while (turn >= n_units) turn -= n_units;  // at most five times
+  return turn;
+}
+
 }  // namespace
 
-// Grid: n_chunks * B * Hkv workgroups of NW waves, chunk-major.  Partial rows are indexed
+// Grid: (B * Hkv units, n_chunks), workgroups of NW waves.  Partial rows are indexed
 // (b * Hq + h) * Tq + i, each with n_chunks slots.
-template <int D, int NW>
+// SPLIT: several chunks; a call of one has no part in that logic (a branch on the length before
+// the other loads cost 0.6 of 5.6 us with a short cache).
+template <int D, int NW, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
     const bf16 *__restrict__ Q, const bf16 *__restrict__ Kc, const bf16 *__restrict__ Vc,
     const int *__restrict__ cache_seqlens, bf16 *__restrict__ O, float *__restrict__ LSE,
     float *__restrict__ part_o, float *__restrict__ part_ml, int B, int Hq, int Hkv, int Tq,
-    int Lmax, int n_chunks, float scale_log2) {
+    int Lmax, int n_chunks, int log2_min, float scale_log2) {
   using P = DecShape<D>;
   constexpr int KK = P::KK, DB = P::DB, CH = P::CH;
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
   bf16 (*lds)[P::WAVE_LDS] = reinterpret_cast<bf16 (*)[P::WAVE_LDS]>(smem);
   __shared__ float wm[NW][32], wsum[NW][32];
-  const int n_units = B * Hkv;
-  const int chunk = blockIdx.x / n_units, bhk = blockIdx.x - chunk * n_units;
+  const int chunk = SPLIT ? blockIdx.y : 0;
+  int bhk = blockIdx.x;
+  // B * Hkv is the grid's width; reading gridDim instead would put 256 bytes of hidden
+  // arguments on every launch (1 us of a short call).
+  if (const int n_units = B * Hkv; SPLIT && n_units >= 8) {
+    bhk -= chunk_turn(chunk, n_units);
+    if (bhk < 0) bhk += n_units;
+  }
   const int b = bhk / Hkv, hk = bhk - b * Hkv;
   const int G = Hq / Hkv, R = G * Tq;
   const int wave = wave_id(), lane = threadIdx.x & 63;
@@ -148,10 +190,10 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
   const int pos = L - Tq + i;  // last visible key of this column
   const int64_t qrow = ((int64_t)b * Hq + h) * Tq + i;
 
-  // The unit's blocks in use are dealt evenly to its chunks, a chunk's blocks to its waves
-  // in turn, so every workgroup of a unit has the same work whatever the cache length.
-  const int nb = (L + kDecBlock - 1) / kDecBlock, per = (nb + n_chunks - 1) / n_chunks;
-  const int blk0 = chunk * per + wave, blk1 = min((chunk + 1) * per, nb);
+  // The unit's blocks in use, in turn over all waves of its workgroups.
+  const int nb = (L + kDecBlock - 1) / kDecBlock;
+  const int used = SPLIT ? used_chunks(nb, n_chunks, log2_min) : 1, step = used * NW;
+  const int blk0 = chunk < used ? chunk * NW + wave : nb;
   bf16 *wl = lds[wave];
 
   f32x16 oacc[DB];
@@ -159,7 +201,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
   for (int db = 0; db < DB; ++db) oacc[db] = f32x16{};
   float m_t = -INFINITY, l_part = 0.f;
 
-  if (blk0 < blk1) {
+  if (blk0 < nb) {
     const int64_t kvbase = ((int64_t)b * Hkv + hk) * Lmax * D;
     uint32_t koff[P::LOADS], voff[P::LOADS];  // this lane's byte offsets within a 32-row block
 #pragma unroll
@@ -168,47 +210,53 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
       koff[j] = (uint32_t)(row * D + swz_l<D, 1>(row, pc) * 8) * 2;
       voff[j] = (uint32_t)(row * D + swz<D>(row, pc) * 8) * 2;
     }
-    auto load_block = [&](int k0, int stage) {  // rows k0..k0+31 of K and V -> an LDS stage
-      bf16 *dst = wl + stage * 2 * kDecBlock * D;
-      const int64_t at = kvbase + (int64_t)k0 * D;
-      const uint32_t left = (uint32_t)(L - k0) * D * 2;  // keys >= L read as zero
-      const auto rk = make_rsrc(Kc + at, left), rv = make_rsrc(Vc + at, left);
+    auto load = [&](const bf16 *src, const uint32_t (&off)[P::LOADS], bf16 *dst, int k0) {
+      const auto rs = make_rsrc(src + kvbase + (int64_t)k0 * D, (uint32_t)(L - k0) * D * 2);
 #pragma unroll
-      for (int j = 0; j < P::LOADS; ++j) {
-        buf_load16_lds(rk, koff[j], dst + 64 * j * 8);
-        buf_load16_lds(rv, voff[j], dst + kDecBlock * D + 64 * j * 8);
-      }
+      for (int j = 0; j < P::LOADS; ++j) buf_load16_lds(rs, off[j], dst + 64 * j * 8);
     };
+    bf16 *Kt = wl, *Vt = wl + kDecBlock * D;
     bf16x8 qf[KK];
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk)
       qf[kk] = *reinterpret_cast<const bf16x8 *>(Q + qrow * D + 16 * kk + 8 * lg);
 
-    load_block(blk0 * kDecBlock, 0);
+    load(Kc, koff, Kt, blk0 * kDecBlock);
+    load(Vc, voff, Vt, blk0 * kDecBlock);
     const int first_masked = L - Tq;  // keys past this need the mask for some column
-    int stage = 0;
 #pragma unroll 1
-    for (int blk = blk0; blk < blk1; blk += NW, stage ^= 1) {
-      const int k0 = blk * kDecBlock;
-      if (blk + NW < blk1) {
-        load_block(k0 + NW * kDecBlock, stage ^ 1);
-        wait_vmcnt<P::VMEM_PER_BLOCK>();  // this block's K and V are in
-      } else {
-        wait_vmcnt<0>();
-      }
+    for (int blk = blk0; blk < nb; blk += step) {
+      const int k0 = blk * kDecBlock, kn = k0 + step * kDecBlock;
+      const bool more = blk + step < nb;
+      wait_vmcnt<P::LOADS>();  // this block's K is in; its V may be in flight
       __builtin_amdgcn_sched_barrier(0);
-      const bf16 *Kt = wl + stage * 2 * kDecBlock * D, *Vt = Kt + kDecBlock * D;
+      auto next_k = [&] {
+        if (more) load(Kc, koff, Kt, kn);
+      };
+      auto wait_v = [&] {
+        if (more) wait_vmcnt<P::LOADS>();  // the next K may be in flight, this V is in
+        else wait_vmcnt<0>();
+      };
       if (k0 + kDecBlock - 1 > first_masked)
-        decode_block<D, true>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
+        decode_block<D, true>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane, next_k, wait_v);
       else
-        decode_block<D, false>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane);
+        decode_block<D, false>(Kt, Vt, qf, oacc, m_t, l_part, scale_log2, k0, pos, L, lane, next_k, wait_v);
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the V rows are read
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) load(Vc, voff, Vt, kn);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
 
+  if (SPLIT && chunk >= used) {  // an empty partial, whose O the merge does not read
+    if (threadIdx.x < R)
+      *reinterpret_cast<f32x2 *>(part_ml + (qrow * n_chunks + chunk) * 2) = f32x2{-INFINITY, 0.f};
+    return;
+  }
+
   // Merge of the workgroup's waves: every wave scales its partial to the workgroup's running
-  // max and stages it as fp32 rows in its own first stage (its blocks are consumed, its loads
-  // have landed; 32 columns of D floats fill the stage), then the threads add the waves in
+  // max and stages it as fp32 rows in its own stage (its blocks are consumed, its loads have
+  // landed; 32 columns of D floats fill the stage), then the threads add the waves in
   // order.
   const float l = xhalf_sum(l_part);
   if (lg == 0) {
@@ -248,7 +296,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
     }
     const int cg = c / Tq;
     const int64_t row = ((int64_t)b * Hq + hk * G + cg) * Tq + (c - cg * Tq);
-    if (n_chunks == 1) {
+    if (!SPLIT) {
       const float inv = ls == 0.f ? 0.f : 1.f / ls;  // NaN sums reach O and LSE
       *reinterpret_cast<bf16x4 *>(O + row * D + 4 * ch) =
           pack4(t[0] * inv, t[1] * inv, t[2] * inv, t[3] * inv);
@@ -261,7 +309,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
   }
 }
 
-// Merge the n_splits partials of every query row: M = max m over partials with l != 0,
+// Merge the partials of every query row whose unit used several workgroups: M = max m over partials with l != 0,
 // O = sum o_s 2^(m_s - M) / sum l_s 2^(m_s - M), LSE = (M + log2 sum) ln 2; a row with no
 // visible key (every l exactly 0) gets O = 0, LSE = -inf, and a NaN sum makes both NaN.  One 256-thread workgroup per row: thread t sums
 // float4 column t % (D/4) over the partials s = t / (D/4) (mod 256 / (D/4)).  The threads
@@ -271,7 +319,7 @@ __global__ __launch_bounds__(64 * NW) void fa_decode_bf16_kernel(
 template <int D>
 __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
     const float *__restrict__ part_o, const float *__restrict__ part_ml, bf16 *__restrict__ O,
-    float *__restrict__ LSE, int rows, int n_splits) {
+    float *__restrict__ LSE, int n_splits) {
   constexpr int C4 = D / 4, SG = 256 / C4;
   __shared__ float wts[kDecMaxSplits];
   __shared__ float red[8];
@@ -306,8 +354,8 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   f32x4 acc{};
 #pragma unroll 4
   for (int s = sg; s < n_splits; s += SG) {
-    const f32x4 x = po[(int64_t)s * C4];
     const float w = wts[s];
+    const f32x4 x = w != 0.f ? po[(int64_t)s * C4] : f32x4{};  // an unused chunk wrote no O
 #pragma unroll
     for (int e = 0; e < 4; ++e) acc[e] = w != 0.f ? __builtin_fmaf(x[e], w, acc[e]) : acc[e];
   }
@@ -325,70 +373,66 @@ __global__ __launch_bounds__(256) void fa_decode_combine_kernel(
   if (tid == 0) LSE[row] = lsum == 0.f ? -INFINITY : (M + __log2f(lsum)) * kLn2;
 }
 
-// Workgroups per unit and waves per workgroup.
-//  * Enough workgroups to put 128 KB of load stages on every CU (256 of them with four
-//    waves at D = 128, 512 at D = 64), at least one 32-key block per wave: more, smaller
-//    workgroups pay their start and the merge again (32 x 4096 keys, D 128: 90.7 us with
-//    256, 96.2 with 512, 100.0 with 1024; 1 x 16000 keys, 12 heads, D 64: 18.8 with 256,
-//    16.5 with 512).
-//  * Caches of up to 16 blocks (512 keys) run as one chunk, in one launch: 8.3 us at 512
-//    keys, D 128, against 9.3 for four chunks and their merge.
-//  * D = 128 with at most 4096 blocks in all runs two waves per workgroup, at most 256
-//    workgroups: a short call is bound by the start of its workgroups, and two waves merge
-//    sooner (1 x 16384 keys, 8 heads: 19.2 against 19.9 us; 4 x 2000, 2 heads: 9.4 against
-//    10.7).  Above that four waves keep more loads in flight (8 x 8000, 8 heads: 43.2
-//    against 44.6).
-//  * The workgroups of four waves stay within one round of those slots: a few above it ran as
-//    a second, nearly empty round (26 x 2 units, 4818 keys, D 128: 260 workgroups 29.0 us, 208
-//    24.2; 39 x 2, 6721: 312 63.4, 234 52.5; 47 x 2, 2649: 282 30.8, 188 25.3). At D = 64, where
-//    two workgroups share a CU, only where that leaves less than a tenth of the slots empty (14 x 12,
-//    13760: 672 81.5 us, 504 77.8; 16 x 12, 10267 keys of uneven caches: 576 52.1, 384 60.9).
-//    Up to one and a half rounds of D = 128 units of 2048 keys or more are halved, so that the
-//    second round is not one of whole units (36 x 8, 3352: 110.0 -> 102.1; 45 x 8, 5825: 149.5
-//    -> 140.7; but 33 x 8, 1043: 40.2 -> 41.4, and 53 x 8, 4946: 178.6 -> 196.4).
+// Workgroups per unit, waves per workgroup, and the blocks a workgroup takes at least.
+//  * Caches of up to 16 blocks (512 keys) run as one chunk, in one launch: 9.1 us at 512 keys,
+//    D 128, B 1, against 11.0 in two launches for 700.
+//  * Otherwise as many chunks as stay within 512 workgroups, the slots of a device whose CUs hold
+//    two (a few more ran as a second, nearly empty round: 9 x 12 units, 1168 keys, D 64: 540
+//    14.5 us, 432 12.1), or one more where that leaves more than a fifth of the slots empty (16 x 12,
+//    10267 keys of uneven caches, D 64: 384 workgroups 65.7, 576 57.0; 24 x 8, 3000, D 128: 39.8,
+//    36.5, but all full 61.4, 66.5); from one chunk to two only for 2048 keys or more (36 x 8,
+//    3352: 109.4 with one, 100.3 with two; 33 x 8, 1043: 40.1, 40.4, and of uneven caches 20.6,
+//    23.5).  Half as many (256 at D 128) read full caches 1-7% faster and leave a long cache among
+//    short ones to half as many CUs, of 40-60 GB/s each.
+//  * One cache has no others beside it: at D = 128 it takes 256 workgroups (8 heads, 16384
+//    keys: 16.7 us; 512: 17.5).
+//  * D = 128: four waves where a chunk has 24 blocks or more, else two, which merge sooner (26 x 2,
+//    4818 keys, 17 blocks a chunk: 29.9 against 33.7; with 32 blocks, 16 x 8, 4096 keys, four read one
+//    long cache in 17.2 against 23.4, full ones in 52.7 against 51.0).  D = 64: four, and eight
+//    in a call of one chunk of 48 blocks or more (64 x 12, 2000 keys: 69.4 against 72.7; 512 x 12,
+//    512: 142 against 133).
+//  * A chunk's least is its share of a full cache, so that short caches cost one workgroup each; with
+//    up to 32 units, which leave the device idle, a block for every wave (1 x 8, D 128, 1600 of
+//    16384 keys: 8.7 us against 10.7).
 DecodeSplit decode_split(int B, int Hkv, int Lmax, int D) {
   const int64_t units = (int64_t)B * Hkv;
   const int64_t blocks = ((int64_t)Lmax + kDecBlock - 1) / kDecBlock;
-  DecodeSplit s;
-  if (blocks <= 16) {
-    s.n_waves = 4;
-    s.n_chunks = 1;
-    return s;
-  }
-  s.n_waves = D == 128 && units * blocks <= 4096 ? 2 : 4;
-  const int64_t fill = D == 128 ? 256 : 512;
-  const int64_t most = (blocks + s.n_waves - 1) / s.n_waves;
-  int64_t n = (fill + units - 1) / units;
-  if (n > 1 && s.n_waves == 4 && (n - 1) * units >= (D == 128 ? 0 : fill - fill / 10)) {
-    if (n * units > fill) --n;  // one round of the slots
-  } else if (D == 128 && n == 1 && units > fill && 2 * units <= 3 * fill && blocks >= 64) {
-    n = 2;
-  }
-  n = n > most ? most : n;
-  s.n_chunks = (int)(n > kDecMaxSplits ? kDecMaxSplits : n);
-  return s;
+  if (blocks <= 16) return {4, 1, 0};
+  const int64_t slots = B == 1 && D == 128 ? 256 : 512;
+  int64_t n = slots / units;
+  if (n < 1) n = 1;
+  if (n * units < slots * 4 / 5 && (n > 1 || blocks >= 64)) ++n;
+  const bool one = n == 1;
+  int n_waves = D == 64 ? (one && blocks >= 48 ? 8 : 4) : one || blocks / n >= 24 ? 4 : 2;
+  const int64_t most = (blocks + n_waves - 1) / n_waves;
+  n = n > most ? most : n > kDecMaxSplits ? kDecMaxSplits : n;
+  const int64_t least = units <= 32 ? n_waves : (blocks + n - 1) / n;
+  int log2_min = 0;
+  while (least >> (log2_min + 1)) ++log2_min;
+  return {n_waves, (int)n, log2_min};
 }
 
-template <int D, int NW>
+template <int D, int NW, bool SPLIT>
 static hipError_t launch_decode(const void *q, const void *k_cache, const void *v_cache,
                                 const int *cache_seqlens, void *o, float *lse, float *part_o,
                                 float *part_ml, int B, int Hq, int Hkv, int Tq, int Lmax,
-                                int n_chunks, float scale_log2, hipStream_t stream) {
+                                int n_chunks, int log2_min, float scale_log2,
+                                hipStream_t stream) {
   constexpr size_t lds = NW * DecShape<D>::WAVE_LDS * sizeof(bf16);
   // the kernel's static arrays come on top of the dynamic stages
   if (lds + 2 * NW * 32 * sizeof(float) > 65536) {
-    hipError_t e = allow_lds<fa_decode_bf16_kernel<D, NW>>(lds);
+    hipError_t e = allow_lds<fa_decode_bf16_kernel<D, NW, SPLIT>>(lds);
     if (e != hipSuccess) return e;
   }
-  const dim3 grid((unsigned)((int64_t)B * Hkv * n_chunks)), block(64 * NW);
-  fa_decode_bf16_kernel<D, NW><<<grid, block, lds, stream>>>(
+  const dim3 grid((unsigned)((int64_t)B * Hkv), (unsigned)n_chunks), block(64 * NW);
+  fa_decode_bf16_kernel<D, NW, SPLIT><<<grid, block, lds, stream>>>(
       (const bf16 *)q, (const bf16 *)k_cache, (const bf16 *)v_cache, cache_seqlens, (bf16 *)o,
-      lse, part_o, part_ml, B, Hq, Hkv, Tq, Lmax, n_chunks, scale_log2);
+      lse, part_o, part_ml, B, Hq, Hkv, Tq, Lmax, n_chunks, log2_min, scale_log2);
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess || n_chunks == 1) return e;
+  if (e != hipSuccess || !SPLIT) return e;
   const int rows = B * Hq * Tq;
   fa_decode_combine_kernel<D><<<dim3((unsigned)rows), dim3(256), 0, stream>>>(
-      part_o, part_ml, (bf16 *)o, lse, rows, n_chunks);
+      part_o, part_ml, (bf16 *)o, lse, n_chunks);
   return hipGetLastError();
 }
 
@@ -401,10 +445,14 @@ hipError_t launch_decode_bf16(const void *q, const void *k_cache, const void *v_
   float *part_ml = workspace + (int64_t)B * Hq * Tq * sp.n_chunks * D;
   auto go = [&](auto launch) {
     return launch(q, k_cache, v_cache, cache_seqlens, o, lse, part_o, part_ml, B, Hq, Hkv, Tq,
-                  Lmax, sp.n_chunks, scale * kLog2e, stream);
+                  Lmax, sp.n_chunks, sp.log2_min, scale * kLog2e, stream);
   };
-  if (D == 64) return go(launch_decode<64, 4>);
-  return sp.n_waves == 2 ? go(launch_decode<128, 2>) : go(launch_decode<128, 4>);
+  if (sp.n_chunks == 1) {
+    if (D == 64) return sp.n_waves == 8 ? go(launch_decode<64, 8, false>) : go(launch_decode<64, 4, false>);
+    return go(launch_decode<128, 4, false>);
+  }
+  if (D == 64) return go(launch_decode<64, 4, true>);
+  return sp.n_waves == 2 ? go(launch_decode<128, 2, true>) : go(launch_decode<128, 4, true>);
 }
 
 }  // namespace ttfa

@@ -54,10 +54,11 @@ hipError_t launch_bwd_varlen_bf16(const void *q, const void *k, const void *v, c
                                   hipStream_t stream);
 
 // KV-cache decode: q/o [B, Hq, Tq, D], caches [B, Hkv, Lmax, D], lse [B, Hq, Tq],
-// cache_seqlens [B] int32 on the device; workspace of decode_workspace_floats() floats.
+// cache_seqlens [B] int32 on the device; workspace of B * Hq * Tq * n_chunks * (D + 2) floats.
 struct DecodeSplit {
   int n_waves;   // waves per workgroup
-  int n_chunks;  // workgroups per (batch, KV head), one partial per query row each
+  int n_chunks;  // workgroups per (batch, KV head) at most, one partial per query row each
+  int log2_min;  // a workgroup takes 2^log2_min 32-key blocks before the next one gets any
 };
 DecodeSplit decode_split(int B, int Hkv, int Lmax, int D);
 hipError_t launch_decode_bf16(const void *q, const void *k_cache, const void *v_cache,
