@@ -82,6 +82,10 @@ def test_forward_matches_oracle(B, T, Hq, Hkv, D):
     (1, 3, 2, 2, 64),      # fewer rows than one workgroup's groups
     (2, 13, 5, 5, 128),
     (1, 257, 1, 1, 64),    # one row past a backward workgroup, one head: a new table row each
+    (1, 33, 1, 1, 64),     # a partial workgroup: two rows in the first groups, one in the 17th
+    (1, 241, 1, 1, 128),   # two workgroups, the last one's groups of eight, one and no rows
+    (680, 64, 1, 1, 64),   # forward: two rows a group ...
+    (700, 64, 1, 1, 64),   # ... and four
 ])
 def test_row_order_edges(B, T, Hq, Hkv, D):
     test_forward_matches_oracle(B, T, Hq, Hkv, D)

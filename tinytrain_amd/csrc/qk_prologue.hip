@@ -14,7 +14,7 @@
 // Work split: a row is one (b, t, head) vector of D bf16, handled by D/8 lanes holding
 // 8 consecutive elements (16 bytes) each; the RoPE partner of element i (i +- D/2) sits
 // in lane ^ D/16 of the same row group.  A 256-thread workgroup holds 256/(D/8) row groups,
-// each with kRounds (forward) or kBwdRounds (backward) consecutive rows; workgroups are
+// each with up to kRounds (forward) or kBwdRounds (backward) consecutive rows; workgroups are
 // ordered q rows, then k rows, then v rows, each in the inputs' [B, T, H] row order (16-byte
 // loads, whole rows of 128 or 256 bytes).  Consecutive rows of a group are mostly heads of
 // one position, so the group keeps its RoPE table row in registers and counts (b, t, h) up
@@ -49,7 +49,7 @@ namespace ttfa {
 
 namespace {
 
-constexpr int kRounds = 4;      // forward: row-group rounds per workgroup
+constexpr int kRounds = 4;      // forward: rows per lane group, at most (fwd_rounds)
 constexpr int kBwdRounds = 8;   // backward: more rows per workgroup, fewer weight-gradient
                                 // partials for the second kernel to add
 
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256) void qk_prologue_fwd_kernel(
     const float *__restrict__ wq, const float *__restrict__ wk, const Tab *__restrict__ cost,
     const Tab *__restrict__ sint, bf16 *__restrict__ q, bf16 *__restrict__ k,
     bf16 *__restrict__ v, float *__restrict__ rstd_q, float *__restrict__ rstd_k, int B, int T,
-    int Hq, int Hkv, float eps, int nq_wg, int nk_wg) {
+    int Hq, int Hkv, float eps, int rounds, int nq_wg, int nk_wg) {
   using S = PShape<D>;
   constexpr int L = S::L;
   const int lane = threadIdx.x % L, group = threadIdx.x / L;
@@ -159,9 +159,9 @@ __global__ __launch_bounds__(256) void qk_prologue_fwd_kernel(
       wl[i + 4] = b[i];
     }
   }
-  const int64_t row0 = (int64_t)wg * S::ROWS + group * kRounds;
+  const int64_t row0 = ((int64_t)wg * S::GROUPS + group) * rounds;
   if (row0 >= n_rows) return;  // whole row groups leave together
-  const int n = (int)min((int64_t)kRounds, n_rows - row0);
+  const int n = (int)min((int64_t)rounds, n_rows - row0);
   RowWalk at(row0, H, T);
   float c[8], s[8];
   int t_of = -1;  // the position whose table row c and s hold
@@ -246,8 +246,12 @@ __global__ __launch_bounds__(256) void qk_prologue_bwd_kernel(
   }
   float c[8], s[8];
   int t_of = -1;  // the position whose table row c and s hold
-  const int64_t row0 = (int64_t)wg * S::ROWS + group * S::ROUNDS;
-  const int n = (int)max((int64_t)0, min((int64_t)S::ROUNDS, n_rows - row0));
+  // The rows of a last, partial workgroup are spread over all of its groups: eight in a row in
+  // the first ones took a call of 16 rows 10.4 us, one in each 8.2.
+  const int64_t wg_row0 = (int64_t)wg * S::ROWS, wg_rows = min((int64_t)S::ROWS, n_rows - wg_row0);
+  const int per = (int)((wg_rows + S::GROUPS - 1) / S::GROUPS);
+  const int64_t row0 = wg_row0 + group * per;
+  const int n = (int)max((int64_t)0, min((int64_t)per, n_rows - row0));
   RowWalk at(row0, H, T);
   u32x4 g_next, x_next;
   float r_next = 0.f;
@@ -348,11 +352,18 @@ struct Grid {
   int nq, nk, nv;
 };
 
-template <int D, int R = kRounds>
-Grid prologue_grid(int B, int T, int Hq, int Hkv) {
-  const int64_t rows = PShape<D, R>::ROWS;
+Grid prologue_grid(int B, int T, int Hq, int Hkv, int D, int rounds) {
+  const int64_t rows = 256 / (D / 8) * rounds;
   auto n = [&](int H) { return (int)(((int64_t)B * T * H + rows - 1) / rows); };
   return {n(Hq), n(Hkv), n(Hkv)};
+}
+
+// Forward rows per lane group: four, or two where four leave fewer than 1024 workgroups, each a
+// chain of loads and stores (Hq 8, Hkv 2, D 128: 2000 positions 6.5 -> 6.1 us, 4096 8.3 -> 7.2, 8192
+// 11.7 and 11.6, 16384 19.3 and 20.5).
+int fwd_rounds(int B, int T, int Hq, int Hkv, int D) {
+  const Grid g = prologue_grid(B, T, Hq, Hkv, D, kRounds);
+  return (int64_t)g.nq + g.nk + g.nv < 1024 ? kRounds / 2 : kRounds;
 }
 
 int check_prologue(int B, int T, int Hq, int Hkv, int D) {
@@ -360,7 +371,7 @@ int check_prologue(int B, int T, int Hq, int Hkv, int D) {
   if (Hq < 1 || Hkv < 1 || Hq % Hkv != 0) return TTFA_E_GROUP;
   if (B < 1 || T < 1) return TTFA_E_SEQ;
   // workgroup counts must fit the grid
-  const int64_t rows = 256 / (D / 8) * kRounds;
+  const int64_t rows = 256 / (D / 8) * kRounds;  // (two rows a group only below 1024 of them)
   if (((int64_t)B * T * (Hq + 2 * Hkv) + rows - 1) / rows > (int64_t)0x7fffffff) return TTFA_E_SEQ;
   return TTFA_OK;
 }
@@ -393,15 +404,16 @@ int ttfa_qk_prologue_fwd_tables(const void *q_raw, const void *k_raw, const void
   if (!(eps >= 0.f) || !(eps < 1.f)) return TTFA_E_EPS;
   if (table_dtype != TTFA_BF16 && table_dtype != TTFA_F32) return TTFA_E_DTYPE;
   hipStream_t st = static_cast<hipStream_t>(hip_stream);
+  const int rounds = fwd_rounds(B, T, Hq, Hkv, D);
   auto go = [&](auto kern, auto tab, Grid g) {
     using Tab = decltype(tab);
     kern<<<dim3((unsigned)(g.nq + g.nk + g.nv)), dim3(256), 0, st>>>(
         (const bf16 *)q_raw, (const bf16 *)k_raw, (const bf16 *)v_raw, q_norm_w, k_norm_w,
         (const Tab *)cos, (const Tab *)sin, (bf16 *)q, (bf16 *)k, (bf16 *)v, rstd_q, rstd_k, B,
-        T, Hq, Hkv, eps, g.nq, g.nk);
+        T, Hq, Hkv, eps, rounds, g.nq, g.nk);
     return (int)hipGetLastError();
   };
-  const Grid g = D == 64 ? prologue_grid<64>(B, T, Hq, Hkv) : prologue_grid<128>(B, T, Hq, Hkv);
+  const Grid g = prologue_grid(B, T, Hq, Hkv, D, rounds);
   if (table_dtype == TTFA_F32)
     return D == 64 ? go(qk_prologue_fwd_kernel<64, float>, float{}, g)
                    : go(qk_prologue_fwd_kernel<128, float>, float{}, g);
@@ -420,8 +432,7 @@ int ttfa_qk_prologue_fwd(const void *q_raw, const void *k_raw, const void *v_raw
 
 long long ttfa_qk_prologue_workspace_bytes(int B, int T, int Hq, int Hkv, int D) {
   if (check_prologue(B, T, Hq, Hkv, D)) return -1;
-  const Grid g = D == 64 ? prologue_grid<64, kBwdRounds>(B, T, Hq, Hkv)
-                         : prologue_grid<128, kBwdRounds>(B, T, Hq, Hkv);
+  const Grid g = prologue_grid(B, T, Hq, Hkv, D, kBwdRounds);
   return (long long)(g.nq + g.nk) * D * (long long)sizeof(float);
 }
 
@@ -452,8 +463,7 @@ int ttfa_qk_prologue_bwd_tables(const void *dq, const void *dk, const void *dv,
                                                        g.nk);
     return (int)hipGetLastError();
   };
-  const Grid g = D == 64 ? prologue_grid<64, kBwdRounds>(B, T, Hq, Hkv)
-                         : prologue_grid<128, kBwdRounds>(B, T, Hq, Hkv);
+  const Grid g = prologue_grid(B, T, Hq, Hkv, D, kBwdRounds);
   auto dw64 = qk_prologue_dw_kernel<64>, dw128 = qk_prologue_dw_kernel<128>;
   if (table_dtype == TTFA_F32)
     return D == 64 ? go(qk_prologue_bwd_kernel<64, float>, dw64, float{}, g)
