@@ -252,14 +252,14 @@ def test_input_errors_are_loud(bad, msg):
         qp.qk_norm_rope(q, k, v, wq, wk, cos, sin)
 
 
-@pytest.mark.parametrize("i, change, msg", [
-    (0, lambda t: t[:, :, :-1], "dq must be"),
-    (1, lambda t: t.transpose(1, 2), "dk must be"),
-    (2, lambda t: t[:1], "dv must be"),
-    (9, lambda t: t[:, :-1], "rq must be"),
-    (10, lambda t: t.double(), "rk must be"),
+@pytest.mark.parametrize("i, change", [
+    (0, lambda t: t[:, :, :-1]),
+    (1, lambda t: t.transpose(1, 2)),
+    (2, lambda t: t[:1]),
+    (9, lambda t: t[:, :-1]),
+    (10, lambda t: t.double()),
 ])
-def test_backward_refuses_wrong_gradients_and_rstd(i, change, msg):
+def test_backward_refuses_wrong_gradients_and_rstd(i, change):
     """The kernels index every operand by the inputs' shape: anything else is refused on the
     host (the CPU tensors of a well-formed call are refused as such)."""
     q, k, v, wq, wk, cos, sin = _inputs(dtype=torch.bfloat16)
@@ -268,5 +268,5 @@ def test_backward_refuses_wrong_gradients_and_rstd(i, change, msg):
     with pytest.raises(qp.QKPrologueInputError, match="ROCm GPU"):
         qp.qk_norm_rope_bwd(*args)
     args[i] = change(args[i])
-    with pytest.raises(qp.QKPrologueInputError, match=msg):
+    with pytest.raises(qp.QKPrologueInputError, match="dq, dk and dv must be"):
         qp.qk_norm_rope_bwd(*args)

@@ -103,13 +103,17 @@ def _fwd(q_raw, k_raw, v_raw, wq, wk, cos, sin, eps):
 def _bwd(dq, dk, dv, q_raw, k_raw, wq, wk, cos, sin, rq, rk):
     B, T, Hq, D = q_raw.shape
     Hkv = k_raw.shape[2]
-    for name, t, H in (("dq", dq, Hq), ("dk", dk, Hkv), ("dv", dv, Hkv)):
-        if t.shape != (B, H, T, D) or t.device != q_raw.device:
-            raise QKPrologueInputError(f"{name} must be [B, H, T, D] on the inputs' device")
-    for name, t, H in (("rq", rq, Hq), ("rk", rk, Hkv)):
-        if t.shape != (B, T, H) or t.dtype != torch.float32 or t.device != q_raw.device:
-            raise QKPrologueInputError(f"{name} must be the forward's fp32 [B, T, H] rstd")
-    _check(q_raw, k_raw, k_raw, wq, wk, cos, sin)
+    q_shape, k_shape = (B, Hq, T, D), (B, Hkv, T, D)
+    if not (dq.shape == q_shape and dk.shape == k_shape and dv.shape == k_shape
+            and rq.shape == (B, T, Hq) and rk.shape == (B, T, Hkv)
+            and rq.dtype == rk.dtype == torch.float32
+            and dq.device == dk.device == dv.device == rq.device == rk.device == q_raw.device):
+        raise QKPrologueInputError(
+            "dq, dk and dv must be [B, H, T, D] and rq and rk the forward's fp32 [B, T, H] rstd, "
+            "on the inputs' device")
+    if not (q_raw.is_cuda and q_raw.is_contiguous() and k_raw.is_contiguous()
+            and q_raw.dtype == k_raw.dtype == torch.bfloat16):
+        _check(q_raw, k_raw, k_raw, wq, wk, cos, sin)   # raises
     dev = q_raw.device
     ct, st, tab = _tables(cos, sin, T, dev)
     wq32, wk32 = wq.float().contiguous(), wk.float().contiguous()
