@@ -730,7 +730,7 @@ def _prologue_bench(dev, steps: int, warmup: int, settle_ms: float = 0.0) -> int
         "fused": {"fwd_ms": round(fused_fwd, 4), "bwd_ms": round(fused_bwd, 4),
                   "note": "C ABI calls (kernels only; bwd = main pass + weight-gradient sum)"},
         "fused_op": {"fwd_ms": round(op_fwd, 4), "bwd_ms": round(op_bwd, 4),
-                     "note": "torch custom op: adds the bf16 table conversion and allocation"},
+                     "note": "torch custom op: adds the dispatch and the allocations (fp32 tables)"},
         "eager_torch": {"fwd_ms": round(eager_fwd, 4), "bwd_ms": round(eager_bwd_ms, 4),
                         "note": "model.py:83-93 expressions: norm, transpose, apply_rope, "
                                 ".contiguous(); backward through autograd"},

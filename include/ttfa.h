@@ -94,13 +94,18 @@ int ttfa_bwd(const void *q, const void *k, const void *v, const void *o,
 
 /*
  * ttfa_bwd with a larger workspace: ttfa_bwd_workspace_bytes(...) bytes (-1 for an invalid
- * shape), 16-byte aligned, overwritten.  Where one workgroup per 128 keys of a KV head
- * would leave most of the device idle (few KV heads and a small batch), the dK/dV pass
- * deals each key tile's work to several workgroups, whose fp32 partial sums in the
- * workspace a further launch adds in a fixed order: still no atomics, bitwise
- * reproducible, but rounded in another order than ttfa_bwd.  For every other shape it is
- * ttfa_bwd.  A single sequence (B = 1) is split only at D = 128 and T > 1792, so that it
- * keeps the bits of ttfa_varlen_bwd below.
+ * shape), 16-byte aligned, overwritten.  The size is that of this very shape: it changes
+ * with the split and may grow as B or T shrinks, so a buffer kept for several shapes needs
+ * the largest of their sizes, not the size of the largest shape.
+ *
+ * Where one workgroup per key tile (128 keys of a KV head in bf16, 16 in fp32) would leave
+ * most of the device idle (few KV heads and a small batch), the dK/dV pass deals a key
+ * tile's work to several workgroups, whose fp32 partial sums in the workspace a further
+ * launch adds in a fixed order: still no atomics, bitwise reproducible, but rounded in
+ * another order than ttfa_bwd.  For every other shape it is ttfa_bwd.  bf16 splits a single
+ * sequence (B = 1) only at D = 128 and T > 1792: elsewhere its dK and dV keep the bits of
+ * ttfa_varlen_bwd below.  fp32, which has no packed form, splits at any B where a key tile's
+ * list (query heads x row blocks) is far longer than an even share of the launch.
  */
 long long ttfa_bwd_workspace_bytes(int B, int Hq, int Hkv, int T, int D, int dtype);
 
@@ -174,7 +179,9 @@ int ttfa_bwd_dkdv(const void *q, const void *k, const void *v, const void *dout,
  *                    written.
  * Validation as above, plus TTFA_E_DTYPE for anything but TTFA_BF16 and TTFA_E_SEQ
  * for n_seq, total or max_seqlen < 1.  Results for each sequence are bitwise those of
- * ttfa_fwd / ttfa_bwd on that sequence alone (B = 1, T = its length).
+ * ttfa_fwd / ttfa_bwd on that sequence alone (B = 1, T = its length), except where that
+ * call runs a 256-row kernel: O and LSE at D = 128, T > 3840 and dQ at D = 128, T > 1792,
+ * each with at least 256 pairs of 256-row tiles.
  */
 int ttfa_varlen_fwd(const void *q, const void *k, const void *v, void *o, float *lse,
                     const int *cu_seqlens, int n_seq, int total, int max_seqlen, int Hq, int Hkv,
@@ -200,7 +207,9 @@ int ttfa_varlen_bwd(const void *q, const void *k, const void *v, const void *o,
  *                       to 0 .. max_seqlen; a row that sees no key gets O = 0, LSE = -inf
  *   lse               : [B, Hq, Tq] fp32 out (natural log)
  *   workspace         : ttfa_decode_workspace_bytes(...) bytes, 16-byte aligned (fp32
- *                       per-split partials; overwritten)
+ *                       per-split partials; overwritten).  The size is that of this very
+ *                       shape and may grow as B or max_seqlen shrinks: a buffer kept for
+ *                       several shapes needs the largest of their sizes.
  * Supported: D in {64, 128}, Hq % Hkv == 0, (Hq / Hkv) * Tq <= 32 (TTFA_E_QROWS),
  * B, Tq, max_seqlen >= 1.  One launch on hip_stream, or two (split pass, merge pass) where
  * the keys of a head are split over workgroups.

@@ -2,7 +2,8 @@
 
 Plain eager calls must give exactly what the custom ops give, gradients included, and
 everything else must still reach the custom ops: dispatch modes, functorch, forward-mode
-tangents, recorded backwards and inputs outside the contract.
+tangents, recorded backwards and inputs outside the contract.  Tracing by torch.compile is
+covered without a GPU in test_compile_host.py.
 """
 
 import pytest

@@ -452,8 +452,10 @@ static hipError_t launch_dkdv(const void *q, const void *k, const void *v, const
 // outweigh 240 partials more than there are: 24x12/4x129 (6 -> 2 stages, 480 partials) would be
 // 25.1 -> 31.7 us, 8x4/4x800 (7 -> 2, 512) 34.0 -> 39.9, 2x12/12x900 (8 -> 2, 480) 37.0 -> 41.5;
 // 12x12/4x400 (12 -> 3, 480) is 40.5 -> 38.4, 16x8/2x129 (8 -> 2, 192) 25.5 -> 23.0.
-// A single sequence keeps the unsplit sums, the bits of the packed entry point, except at
-// D = 128 above T = 1792, where those differ by the 256-row kernels too.
+// A single sequence keeps the unsplit sums, so its dK and dV have the packed entry point's bits,
+// except at D = 128 above T = 1792: there the split halves the backward (939 -> 513 us above)
+// and dK and dV differ from the packed ones by the order of their sums (dQ does only where the
+// 256-row kernel takes it).
 DkdvSplit dkdv_split(int B, int Hq, int Hkv, int T, int D) {
   const DkdvSplit none{0, 0, 0};
   if (B == 1 && !(D == 128 && T > 1792)) return none;

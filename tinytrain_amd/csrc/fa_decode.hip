@@ -30,9 +30,10 @@
 // registers, 32 bytes from each of 32 rows per instruction, read 8% slower at 32 x 4096 keys.
 // Per block: S^T = K Q^T, online softmax in the exp2 domain (lazy rescale as in the forward
 // kernel), O^T += V^T P^T.  The waves' partials (unnormalised O, running max m in log2 units,
-// sum l) are merged through LDS, in wave order.  A unit with one workgroup has its O and LSE
-// written by it; otherwise each writes one fp32 partial per query row, and a second kernel
-// merges the chunks with the log-sum-exp rule.
+// sum l) are merged through LDS, in wave order.  In a call of one chunk the workgroup writes its
+// unit's O and LSE; otherwise each writes one fp32 partial per query row (an empty one where the
+// unit's cache leaves it no blocks), and a second kernel merges all chunks with the log-sum-exp
+// rule.
 //
 // What bounds it: the cache bytes from HBM (a plain read kernel reaches 6.8-7.1 TB/s on
 // MI355X), for small caches the launches, and for one long cache among short ones the rate of
