@@ -462,34 +462,38 @@ __device__ __forceinline__ void dkdv_block(float *lds, const F32Bwd &a, int bhk,
     const int g = i / per_g, qb = kb + (i - g * per_g), q0 = qb * kF32Rows;
     float delta[4], lse[4];
     store_block<D>(tdo, nxt.dout, lane);
-    float qa[D / 4], doa[D / 4];
+    float qa[D / 4], doa[D / 4], oa[OWN_DELTA ? D / 4 : 1];
     read_rowfrag<D>(doa, tdo, j, n);
     if constexpr (OWN_DELTA) {
-      // Delta of row q0 + n in every lane of column n, then row q0 + 4 j + r from lane 4 j + r
-      // (O passes through the Q tile, as in dq_block: a third tile per wave and O held with
+      // O passes through the Q tile, as in dq_block: a third tile per wave and O held with
       // the other prefetches cost 69.1 us against 66.9 at 2x8/2x500 D = 128, 81.3 against 78.9
-      // at 2x12/4x700 D = 64).
-      float oa[D / 4];
+      // at 2x12/4x700 D = 64.
       store_block<D>(tq, nxt.o, lane);
       read_rowfrag<D>(oa, tq, j, n);
-      float d = 0.f;
-#pragma unroll
-      for (int e = 0; e < D / 4; ++e) d = __builtin_fmaf(oa[e], doa[e], d);
-      d = group_sum(d);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) delta[r] = __shfl(d, 4 * j + r);
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) delta[r] = nxt.delta[r];
     }
 #pragma unroll
     for (int r = 0; r < 4; ++r) lse[r] = nxt.lse[r];
+    if constexpr (!OWN_DELTA) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) delta[r] = nxt.delta[r];
+    }
     store_block<D>(tq, nxt.q, lane);
     if (i + NW < n_items) load_item(nxt, i + NW);  // in flight during this item's products
     read_rowfrag<D>(qa, tq, j, n);
     // S and dP: register r = query q0 + 4 j + r, key k0 + n.
     const f32x4 s = dot_block<D>(qa, kf);
     const f32x4 dp = dot_block<D>(doa, vf);
+    if constexpr (OWN_DELTA) {
+      // Delta of row q0 + n in every lane of column n, then row q0 + 4 j + r from lane 4 j + r.
+      // Formed here, beside the products, not before them, where it lengthened every item's
+      // chain: 1x8/2x100 D = 64 14.30 -> 13.85 us, 2x2/2x437 14.96 -> 14.35, 2x12/4x700 79.5 -> 78.5.
+      float d = 0.f;
+#pragma unroll
+      for (int e = 0; e < D / 4; ++e) d = __builtin_fmaf(oa[e], doa[e], d);
+      d = group_sum(d);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) delta[r] = __shfl(d, 4 * j + r);
+    }
     f32x4 p, ds;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
